@@ -16,17 +16,24 @@
 //    of at most 8 bits, exact in bf16.  So every product of v_mfma_f32_32x32x16_bf16 is exact
 //    and only the fp32 sums round, as in the reference's fp32 loop (in another order).  The
 //    terms go in smallest first: lo, mid, hi.
-//  * The K loop steps over two 32-element blocks.  Per block, six MFMAs (two 16-element halves
-//    x three terms) give the block's partial sum P = sum_k a_k q_k for a 32 x 32 patch, then
-//    acc = fma(d_w, P, acc): one VALU op per output and block (the reference multiplies d_w into
-//    every weight element instead; the same value up to rounding).
-//  * Staging: the activation tile is converted to the three bf16 planes and the weight quants
-//    to bf16 once per workgroup and K step, into LDS (row pitch 144 bytes: the 16-byte fragment
-//    reads of 16 consecutive rows hit distinct banks).  The next step's global loads are issued
-//    into registers before the current step's MFMAs.
-//  * Tiles: 128 x 128 (four waves of 64 x 64) for M > 32; 32 x 128 (four waves side by side)
-//    for M <= 32.  Grids below 256 workgroups are split along K; the partial sums are added in
-//    split order by the int8 GEMM's split-K reduction (deterministic).
+//  * Per 32-element block, six MFMAs (three terms x two 16-element halves) give the block's partial
+//    sum P = sum_k a_k q_k for a 32 x 32 patch, then acc = fma(d_w, P, acc): one VALU op per output
+//    and block (the reference multiplies d_w into every weight element instead; the same value up
+//    to rounding).
+//  * The activations are split and the weight quants converted once per workgroup and block, into
+//    LDS in fragment order: a wave's 16-byte reads are lane-linear, without bank conflicts.  Two
+//    buffers: block k + 1 is converted between the MFMAs of block k, one barrier per block.
+//  * Tiles of 128 x 256 (eight waves of 64 x 64), 128 x 128 (four) and 64 x 128 (four of 32 x 64),
+//    chosen with the number of K splits by a cost model over the grid (w16_plan); the split partial
+//    sums are added in split order by the int8 GEMM's split-K reduction (deterministic).
+//  * Bound: the chip's power.  Six MFMAs take 198 cycles per patch and block, and at full rate with
+//    random operands the clock falls from 2.4 to about 2 GHz; every instruction beside them costs
+//    time.  M = 2048, N = K = 4096, Q4_0: 183 us (343 TFLOP/s of fp32-exact products, 1.03 PFLOP/s
+//    on the bf16 pipe), of it 138 the MFMAs with their LDS reads alone, 12 the epilogue and about
+//    35 the conversions (230 us on single-buffered 128 x 128 tiles with 144-byte row pitch and two
+//    barriers per two blocks).  M = 395, N = 3871, K = 1344: 25.4 us (65.5).
+//  * Measured, level or slower: three buffers with the next block's first fragments read ahead of
+//    the barrier, and activation loads four blocks ahead (187-195 us).
 //  * Rows / columns past M or N load a clamped in-range row and are not stored.
 #include "ksq_device.h"
 #include "ksq_internal.h"
@@ -35,22 +42,28 @@ namespace ksq {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
+// BM x BN workgroup tile, waves of 32 TM x 32 TN.  Two threads per weight row stage the weights.
 template <int BM_, int BN_, int TM_, int TN_>
 struct W16Tile {
     static constexpr int BM = BM_, BN = BN_, TM = TM_, TN = TN_;
     static constexpr int WN = BN / (32 * TN);   // waves along N
     static constexpr int WM = BM / (32 * TM);   // waves along M
-    static_assert(WN * WM == 4, "four waves per workgroup");
-    static_assert(BN == 128, "the weight staging maps 128 rows x 2 blocks onto 256 threads");
-    static_assert(BM % 16 == 0 && BM * 16 % 256 == 0, "the activation staging maps 16 float4 per row");
+    static constexpr int NT = 64 * WN * WM;     // threads per workgroup
+    static constexpr int AC = (BM * 4 + NT - 1) / NT;   // 8-float activation chunks per thread and block
+    static_assert(NT == 2 * BN, "a thread stages half a weight block per row");
 };
+using W16Huge = W16Tile<128, 256, 2, 2>;
 using W16Big = W16Tile<128, 128, 2, 2>;
-using W16Skinny = W16Tile<32, 128, 1, 1>;
-
-constexpr int kW16Pitch = 72;         // bf16 per staged row: 64 values of the step + 8 padding
+using W16Mid = W16Tile<64, 128, 1, 2>;
 
 typedef float f32x2v __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x3a4 __attribute__((ext_vector_type(3), aligned(4)));
+
+template <int V>
+struct W16Int {
+    static constexpr int value = V;
+};
 
 // Two fp32 values as a bf16 pair (round to nearest even), lo in the low half: one packed
 // conversion (v_cvt_pk_bf16_f32) instead of two single ones and the shift and or that merge them.
@@ -59,6 +72,262 @@ __device__ __forceinline__ uint32_t bf16_pair(float lo, float hi) {
 }
 __device__ __forceinline__ float bf16_low_f32(uint32_t p) { return __builtin_bit_cast(float, p << 16); }
 __device__ __forceinline__ float bf16_high_f32(uint32_t p) { return __builtin_bit_cast(float, p & 0xFFFF0000u); }
+
+// The four nibbles at bits 0, 8, 16, 24 of w, less 8, as two bf16 pairs.
+__device__ __forceinline__ u32x2 w16_nibbles(uint32_t w) {
+    float q[4];
+#pragma unroll
+    for (int b = 0; b < 4; b++) q[b] = __builtin_amdgcn_cvt_off_f32_i4((int)(w >> (8 * b)));
+    return u32x2{bf16_pair(q[0], q[1]), bf16_pair(q[2], q[3])};
+}
+__device__ __forceinline__ u32x2 w16_bytes(uint32_t w) {
+    float q[4];
+#pragma unroll
+    for (int b = 0; b < 4; b++) q[b] = (float)(int8_t)((w >> (8 * b)) & 0xFFu);
+    return u32x2{bf16_pair(q[0], q[1]), bf16_pair(q[2], q[3])};
+}
+
+// WT: kWQ40 or kWQ80.  W: [N][K/32] blocks (4-byte aligned); A: fp32 [M][K] (16-byte aligned);
+// C: fp32 [M][N], or split z's partial [M][N] at C + z*M*N.  nb = K/32, even.
+// Workgroup x is a linear tile index whose tiles each XCD takes as one contiguous run in
+// row-major tile order (xcd_tile): whole rows of tiles per XCD, so each XCD's L2 fetches its
+// activation rows once (the plain grid spreads each row's column tiles over all 8 XCDs).
+template <class T, int WT>
+__global__ __launch_bounds__(T::NT, 2) void w16_kernel(const uint8_t* __restrict__ W, const float* __restrict__ A,
+                                                       float* __restrict__ C, int M, int N, int nb) {
+    constexpr int BM = T::BM, BN = T::BN, TM = T::TM, TN = T::TN, NT = T::NT, AC = T::AC;
+    constexpr int BB = block_bytes(WT);                    // 18 or 34
+    constexpr int WW = (WT == kWQ40) ? 6 : 10;             // weight dwords a thread loads per two blocks
+    // fragment order: [32-row group][term: lo, mid, hi][16-element half][lane][8 bf16]
+    constexpr int ABytes = BM * 32 * 2 * 3, WBytes = BN * 32 * 2;
+    // two buffers: block k + 1 is staged while block k is multiplied
+    constexpr int DBytes = 2 * BN * 4, Buf = ABytes + WBytes + DBytes;
+    __shared__ __attribute__((aligned(16))) uint8_t sm[2 * Buf];
+
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int wm = wave / T::WN, wn = wave % T::WN;
+    const int l32 = lane & 31, hi = lane >> 5;
+    const int gn = (N + BN - 1) / BN, tiles = gn * ((M + BM - 1) / BM);
+    const int L = xcd_tile((int)blockIdx.x, (int)gridDim.x);
+    if (L >= tiles) return;   // padding of the grid to a multiple of 8 (whole workgroup)
+    const int m0 = (L / gn) * BM, n0 = (L % gn) * BN;
+
+    // split z covers K steps [s_lo, s_hi) of two blocks each
+    const int nsteps = nb / 2, Z = (int)gridDim.z, z = (int)blockIdx.z;
+    const int s_lo = (int)((long long)nsteps * z / Z), s_hi = (int)((long long)nsteps * (z + 1) / Z);
+    C += (size_t)z * (size_t)M * (size_t)N;
+    const size_t K = (size_t)nb * 32;
+
+    // ---- staging assignment ----
+    // activations: chunk c = t + NT i is the 8 floats at 8 (c % 4) of row c / 4 (four lanes read a
+    // row's 128-byte segment); weights: row t % BN, half t / BN (wave-uniform) of its blocks
+    const float* asrc[AC];
+    uint32_t adst[AC];
+#pragma unroll
+    for (int i = 0; i < AC; i++) {
+        const int c = t + NT * i, r = c >> 2, q = c & 3;
+        asrc[i] = A + (size_t)min(m0 + min(r, BM - 1), M - 1) * K + 8 * q;
+        // rows of a fragment are XORed with twice the chunk number: the 8 lanes of a write (2 rows
+        // x 4 chunks, whose fragments lie multiples of 512 bytes apart) then hit 8 bank groups
+        adst[i] = (uint32_t)((r >> 5) * 6144 + (q >> 1) * 1024 + (q & 1) * 512 + (((r & 31) ^ (2 * q)) << 4));
+    }
+    const bool a_on = BM * 4 >= NT || t < BM * 4;
+    const int wr = t % BN, wh = t / BN;
+    const uint8_t* wrow = W + (size_t)min(n0 + wr, N - 1) * nb * BB;
+    f32x4 pa[2][AC][2];        // blocks k + 1 and k + 2 while block k is multiplied
+    uint32_t pw[WW];           // the weights of two blocks
+    auto load_a = [&](auto bv, int kb) __attribute__((always_inline)) {
+        constexpr int b = decltype(bv)::value;
+        if (a_on) {
+#pragma unroll
+            for (int i = 0; i < AC; i++) {
+                pa[b][i][0] = *(const f32x4*)(asrc[i] + (size_t)kb * 32);
+                pa[b][i][1] = *(const f32x4*)(asrc[i] + (size_t)kb * 32 + 4);
+            }
+        }
+    };
+    // the weight bytes of step s (two blocks) that this thread converts.  Q4_0 (36 bytes: d at 0
+    // and 18, quants at 2 and 20): half h is quant bytes 8h .. 8h + 7, i.e. dwords 2h .. 2h + 2 and
+    // 4 + 2h .. 6 + 2h.  Q8_0 (68 bytes: d at 0 and 34, quants at 2 and 36): half h is bytes
+    // 16h .. 16h + 15, i.e. dwords 4h .. 4h + 4 and 8 + 4h .. 12 + 4h.
+    auto load_w = [&](int s) __attribute__((always_inline)) {
+        const uint32_t* src = (const uint32_t*)(wrow + (size_t)s * 2 * BB);
+        if constexpr (WT == kWQ40) {
+            const u32x3a4 x = *(const u32x3a4*)(src + 2 * wh), y = *(const u32x3a4*)(src + 4 + 2 * wh);
+            pw[0] = x.x; pw[1] = x.y; pw[2] = x.z;
+            pw[3] = y.x; pw[4] = y.y; pw[5] = y.z;
+        } else {
+            const u32x4a4 x = *(const u32x4a4*)(src + 4 * wh), y = *(const u32x4a4*)(src + 9 + 4 * wh);
+            pw[0] = x.x; pw[1] = x.y; pw[2] = x.z; pw[3] = x.w; pw[4] = src[4 * wh + 4];
+            pw[5] = src[8 + 4 * wh];
+            pw[6] = y.x; pw[7] = y.y; pw[8] = y.z; pw[9] = y.w;
+        }
+    };
+    // chunk i of the activation block in pa[b], as three bf16 terms, into buffer b
+    auto store_a = [&](auto bv, int i, uint8_t* buf) __attribute__((always_inline)) {
+        constexpr int b = decltype(bv)::value;
+        if (a_on) {
+            uint32_t ph[4], pm[4], pl[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const float a0 = pa[b][i][j >> 1][2 * (j & 1)], a1 = pa[b][i][j >> 1][2 * (j & 1) + 1];
+                ph[j] = bf16_pair(a0, a1);
+                const float r0 = a0 - bf16_low_f32(ph[j]), r1 = a1 - bf16_high_f32(ph[j]);
+                pm[j] = bf16_pair(r0, r1);
+                pl[j] = bf16_pair(r0 - bf16_low_f32(pm[j]), r1 - bf16_high_f32(pm[j]));
+            }
+            uint8_t* d = buf + adst[i];
+            *(u32x4*)d = u32x4{pl[0], pl[1], pl[2], pl[3]};
+            *(u32x4*)(d + 2048) = u32x4{pm[0], pm[1], pm[2], pm[3]};
+            *(u32x4*)(d + 4096) = u32x4{ph[0], ph[1], ph[2], ph[3]};
+        }
+    };
+    // block b of the step in pw into weight buffer b
+    auto store_w = [&](auto bv, uint8_t* buf) __attribute__((always_inline)) {
+        constexpr int b = decltype(bv)::value;
+        uint8_t* d = buf + ABytes + (wr >> 5) * 2048 + ((wr & 31) << 4);
+        float* sd = (float*)(buf + ABytes + WBytes);   // the second BN: from the half that holds no scale, never read
+        if constexpr (WT == kWQ40) {
+            const uint32_t q0 = b ? pw[4] : word_at(pw, 2), q1 = b ? pw[5] : word_at(pw, 6);
+            const uint32_t x0 = q0 ^ 0x88888888u, x1 = q1 ^ 0x88888888u;
+            const u32x2 l0 = w16_nibbles(x0), l1 = w16_nibbles(x1);
+            const u32x2 h0 = w16_nibbles(x0 >> 4), h1 = w16_nibbles(x1 >> 4);
+            *(u32x4*)(d + 512 * wh) = u32x4{l0.x, l0.y, l1.x, l1.y};          // elements 8h ..
+            *(u32x4*)(d + 1024 + 512 * wh) = u32x4{h0.x, h0.y, h1.x, h1.y};   // elements 16 + 8h ..
+            sd[t] = 16.0f * f16_to_f32(b ? pw[3] >> 16 : pw[0] & 0xFFFFu);
+        } else {
+            u32x2 v[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = w16_bytes(b ? pw[6 + j] : word_at(pw, 2 + 4 * j));
+            *(u32x4*)(d + 1024 * wh) = u32x4{v[0].x, v[0].y, v[1].x, v[1].y};        // elements 16h ..
+            *(u32x4*)(d + 1024 * wh + 512) = u32x4{v[2].x, v[2].y, v[3].x, v[3].y};  // 16h + 8 ..
+            sd[t] = f16_to_f32(b ? pw[5] >> 16 : pw[0] & 0xFFFFu);
+        }
+    };
+
+    f32x16 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
+    f32x16 zero;
+#pragma unroll
+    for (int r = 0; r < 16; r++) zero[r] = 0.0f;
+    // byte offset of this lane's slot in half h of a fragment (chunk q = 2h + hi)
+    uint32_t aoff[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+        aoff[h] = (uint32_t)(wm * TM * 6144 + h * 1024 + hi * 512 + ((l32 ^ (2 * (2 * h + hi))) << 4));
+    const uint32_t woff = (uint32_t)(wn * TN * 2048 + lane * 16);
+
+    // Block b (buffer b) times its weights, with the staging of the next block (`stage`) in the same
+    // straight-line code: the scheduling groups put its conversions between the MFMAs
+    auto compute = [&](const uint8_t* buf, auto stage) __attribute__((always_inline)) {
+        bf16x8 wf[TN][2], af[TM][3][2];
+        float dw[TN];
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+#pragma unroll
+            for (int h = 0; h < 2; h++) wf[j][h] = *(const bf16x8*)(buf + ABytes + woff + j * 2048 + h * 1024);
+            dw[j] = *(const float*)(buf + ABytes + WBytes + 4 * (wn * 32 * TN + 32 * j + l32));
+        }
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int e = 0; e < 3; e++)
+#pragma unroll
+                for (int h = 0; h < 2; h++) af[i][e][h] = *(const bf16x8*)(buf + aoff[h] + i * 6144 + e * 2048);
+        stage();
+        f32x16 p[2];
+#pragma unroll
+        for (int u = 0; u <= TM * TN; u++) {
+            if (u < TM * TN) {
+                const int i = u / TN, j = u % TN;
+                // D[m][n]: A operand = activation fragment, B = weights, so a lane holds one column
+                f32x16 c = zero;
+#pragma unroll
+                for (int e = 0; e < 3; e++)
+#pragma unroll
+                    for (int h = 0; h < 2; h++) c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i][e][h], wf[j][h], c, 0, 0, 0);
+                p[u & 1] = c;
+            }
+            if (u > 0) {
+                const int i = (u - 1) / TN, j = (u - 1) % TN;
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[i][j][r] = fmaf(dw[j], p[(u - 1) & 1][r], acc[i][j][r]);
+            }
+        }
+        constexpr int NM = TM * TN * 6;   // MFMAs; per MFMA: a fragment read, 7 vector instructions, an LDS write
+        __builtin_amdgcn_sched_group_barrier(0x100, TN * 3 + 6, 0);
+#pragma unroll
+        for (int k = 0; k < NM; k++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            if (k < 6 * (TM - 1)) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);
+            if (k > NM / 3) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+        }
+    };
+
+    using B0 = W16Int<0>;
+    using B1 = W16Int<1>;
+    uint8_t* const buf0 = sm;
+    uint8_t* const buf1 = sm + Buf;
+    if (s_lo < s_hi) {
+        load_w(s_lo);
+        load_a(B0{}, 2 * s_lo);
+        load_a(B1{}, 2 * s_lo + 1);
+        store_w(B0{}, buf0);
+#pragma unroll
+        for (int i = 0; i < AC; i++) store_a(B0{}, i, buf0);
+    }
+    __syncthreads();
+    for (int s = s_lo; s < s_hi; s++) {
+        const int sn = min(s + 1, s_hi - 1);   // past the last step: staged again, read by nobody
+        load_a(B0{}, 2 * sn);
+        __builtin_amdgcn_sched_barrier(0);   // the loads go out before the block is computed
+        compute(buf0, [&]() __attribute__((always_inline)) {
+            store_w(B1{}, buf1);
+#pragma unroll
+            for (int i = 0; i < AC; i++) store_a(B1{}, i, buf1);
+        });
+        load_w(sn);
+        __syncthreads();
+        load_a(B1{}, 2 * sn + 1);
+        __builtin_amdgcn_sched_barrier(0);   // the loads go out before the block is computed
+        compute(buf1, [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < AC; i++) store_a(B0{}, i, buf0);
+            store_w(B0{}, buf0);
+        });
+        __syncthreads();
+    }
+
+    // lane l holds column n = l % 32 of each 32 x 32 patch, rows m = 8 (r / 4) + 4 (l / 32) + r % 4
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+        const int mb = m0 + (wm * TM + i) * 32 + 4 * hi;
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            const int n = n0 + (wn * TN + j) * 32 + l32;
+            if (n >= N) continue;
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int m = mb + 8 * (r >> 2) + (r & 3);
+                if (m < M) C[(size_t)m * N + n] = acc[i][j][r];
+            }
+        }
+    }
+}
+
+// ---- up to 32 activation rows ----------------------------------------------------------------
+// A 32 x 128 tile, four waves side by side, one LDS buffer of two blocks and the next step's loads
+// in registers.  Bound by the latency of a step, not by the matrix pipe; split along K the plain
+// form is level with or ahead of the double-buffered one (N = K = 4096, M = 8: Q4_0 12.8 vs 13.2
+// us, Q8_0 12.7 vs 14.0; N = 1632, K = 5440, M = 20: 12.6 vs 13.4).
+constexpr int kW16SmallRows = 32;
+constexpr int kW16Pitch = 72;         // bf16 per staged row: 64 values of the step + 8 padding
 
 // 32 weight quants of one block as bf16 into dst (32 values), the block's scale into *d.  v: the
 // dwords holding the block, which starts at byte O of v.
@@ -91,15 +360,11 @@ __device__ __forceinline__ void w16_stage_block(const uint32_t* v, uint16_t* dst
     }
 }
 
-// WT: kWQ40 or kWQ80.  W: [N][K/32] blocks (4-byte aligned); A: fp32 [M][K] (16-byte aligned);
-// C: fp32 [M][N], or split z's partial [M][N] at C + z*M*N.  nb = K/32, even.
-// XG: workgroup x is a linear tile index whose tiles each XCD takes as one contiguous run in
-// row-major tile order (xcd_tile): whole rows of tiles per XCD, so each XCD's L2 fetches its
-// activation rows once (the plain grid spreads each 128-row tile's column tiles over all 8 XCDs).
-template <class T, int WT, bool XG = false>
-__global__ __launch_bounds__(256, 2) void w16_kernel(const uint8_t* __restrict__ W, const float* __restrict__ A,
+// W, A, C and nb as above; grid (column tiles, row tiles, splits).
+template <int WT>
+__global__ __launch_bounds__(256, 2) void w16_small_kernel(const uint8_t* __restrict__ W, const float* __restrict__ A,
                                                      float* __restrict__ C, int M, int N, int nb) {
-    constexpr int BM = T::BM, BN = T::BN, TM = T::TM, TN = T::TN, P = kW16Pitch;
+    constexpr int BM = kW16SmallRows, BN = 128, P = kW16Pitch;
     constexpr int BB = block_bytes(WT);                    // 18 or 34
     constexpr int AC = BM * 16 / 256;                      // activation float4 chunks per thread
     constexpr int WW = (WT == kWQ40) ? 5 : 9;              // weight dwords a thread loads per step
@@ -108,17 +373,8 @@ __global__ __launch_bounds__(256, 2) void w16_kernel(const uint8_t* __restrict__
     __shared__ __attribute__((aligned(16))) float sD[2][BN];
 
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int wm = wave / T::WN, wn = wave % T::WN;
     const int l32 = lane & 31, hi = lane >> 5;
-    int tm = (int)blockIdx.y, tn = (int)blockIdx.x;
-    if constexpr (XG) {
-        const int gn = (N + BN - 1) / BN, tiles = gn * ((M + BM - 1) / BM);
-        const int L = xcd_tile((int)blockIdx.x, (int)gridDim.x);
-        if (L >= tiles) return;   // padding of the grid to a multiple of 8 (whole workgroup)
-        tm = L / gn;
-        tn = L % gn;
-    }
-    const int m0 = tm * BM, n0 = tn * BN;
+    const int m0 = (int)blockIdx.y * BM, n0 = (int)blockIdx.x * BN;
 
     // split z covers K steps [s_lo, s_hi) of two blocks each
     const int nsteps = nb / 2, Z = (int)gridDim.z, z = (int)blockIdx.z;
@@ -167,85 +423,54 @@ __global__ __launch_bounds__(256, 2) void w16_kernel(const uint8_t* __restrict__
         else w16_stage_block<WT, 2>(pw, &sW[wr][32], &sD[1][wr]);
     };
 
-    f32x16 acc[TM][TN];
+    f32x16 acc, zero;
 #pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
-    f32x16 zero;
-#pragma unroll
-    for (int r = 0; r < 16; r++) zero[r] = 0.0f;
-    const bool wave_has_rows = M - m0 - wm * 32 * TM > 0;   // wave-uniform
+    for (int r = 0; r < 16; r++) acc[r] = zero[r] = 0.0f;
+    const int nw = 32 * wave;   // this wave's weight rows of the tile
 
     if (s_lo < s_hi) load(s_lo);
     for (int s = s_lo; s < s_hi; s++) {
         store();
         __syncthreads();
         if (s + 1 < s_hi) load(s + 1);
-        if (wave_has_rows) {
 #pragma unroll
-            for (int kb = 0; kb < 2; kb++) {
-                bf16x8 wf[TN][2], af[3][TM][2];
+        for (int kb = 0; kb < 2; kb++) {
+            bf16x8 wf[2], af[3][2];
 #pragma unroll
-                for (int h = 0; h < 2; h++) {
-                    const int ko = 32 * kb + 16 * h + 8 * hi;
+            for (int h = 0; h < 2; h++) {
+                const int ko = 32 * kb + 16 * h + 8 * hi;
+                wf[h] = *(const bf16x8*)&sW[nw + l32][ko];
 #pragma unroll
-                    for (int j = 0; j < TN; j++) wf[j][h] = *(const bf16x8*)&sW[wn * 32 * TN + 32 * j + l32][ko];
-#pragma unroll
-                    for (int e = 0; e < 3; e++)
-#pragma unroll
-                        for (int i = 0; i < TM; i++) af[e][i][h] = *(const bf16x8*)&sA[e][wm * 32 * TM + 32 * i + l32][ko];
-                }
-#pragma unroll
-                for (int j = 0; j < TN; j++) {
-                    const int nbase = wn * 32 * TN + 32 * j + 4 * hi;
-                    f32x4 dw[4];
-#pragma unroll
-                    for (int q = 0; q < 4; q++) dw[q] = *(const f32x4*)&sD[kb][nbase + 8 * q];
-#pragma unroll
-                    for (int i = 0; i < TM; i++) {
-                        // the MFMA computes D[n][m]: A operand = weight fragment, B = activations
-                        f32x16 p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[j][0], af[0][i][0], zero, 0, 0, 0);
-                        p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[j][1], af[0][i][1], p, 0, 0, 0);
-                        p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[j][0], af[1][i][0], p, 0, 0, 0);
-                        p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[j][1], af[1][i][1], p, 0, 0, 0);
-                        p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[j][0], af[2][i][0], p, 0, 0, 0);
-                        p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[j][1], af[2][i][1], p, 0, 0, 0);
-#pragma unroll
-                        for (int q = 0; q < 4; q++)
-#pragma unroll
-                            for (int r = 0; r < 4; r++)
-                                acc[i][j][4 * q + r] = fmaf(dw[q][r], p[4 * q + r], acc[i][j][4 * q + r]);
-                    }
-                }
+                for (int e = 0; e < 3; e++) af[e][h] = *(const bf16x8*)&sA[e][l32][ko];
             }
+            f32x4 dw[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) dw[q] = *(const f32x4*)&sD[kb][nw + 4 * hi + 8 * q];
+            // the MFMA computes D[n][m]: A operand = weight fragment, B = activations
+            f32x16 p = zero;
+#pragma unroll
+            for (int e = 0; e < 3; e++)
+#pragma unroll
+                for (int h = 0; h < 2; h++) p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[h], af[e][h], p, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[r] = fmaf(dw[r >> 2][r & 3], p[r], acc[r]);
         }
         __syncthreads();
     }
 
     // lane l holds activation row m = l % 32 and weight rows n = 8 (r / 4) + 4 (l / 32) + r % 4
     const bool vec_ok = (N % 4) == 0 && (((uintptr_t)C & 15u) == 0);
+    const int gm = m0 + l32;
+    if (gm >= M) return;
 #pragma unroll
-    for (int i = 0; i < TM; i++) {
-        const int gm = m0 + wm * 32 * TM + 32 * i + l32;
-        if (gm >= M) continue;
+    for (int q = 0; q < 4; q++) {
+        const int gn = n0 + nw + 4 * hi + 8 * q;
+        if (vec_ok && gn + 3 < N) {
+            *(f32x4*)(C + (size_t)gm * N + gn) = f32x4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+        } else {
 #pragma unroll
-        for (int j = 0; j < TN; j++) {
-            const int nbase = n0 + wn * 32 * TN + 32 * j + 4 * hi;
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int gn = nbase + 8 * q;
-                if (vec_ok && gn + 3 < N) {
-                    *(f32x4*)(C + (size_t)gm * N + gn) =
-                        f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-                } else {
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-                        if (gn + r < N) C[(size_t)gm * N + gn + r] = acc[i][j][4 * q + r];
-                }
-            }
+            for (int r = 0; r < 4; r++)
+                if (gn + r < N) C[(size_t)gm * N + gn + r] = acc[4 * q + r];
         }
     }
 }
@@ -415,35 +640,78 @@ constexpr int kW16MinWGs = 256, kW16TargetWGs = 512, kW16MaxSplits = 16;
 constexpr int kW16GemvMaxRows = 4;
 bool w16_uses_gemv(int M) { return M >= 1 && M <= kW16GemvMaxRows; }
 
-bool w16_skinny(int M) { return M <= 32; }
+int w16_tiles(int M, int N, int bm, int bn) { return ((N + bn - 1) / bn) * ((M + bm - 1) / bm); }
 
-int w16_grid_wgs(int M, int N) {
-    const int bm = w16_skinny(M) ? W16Skinny::BM : W16Big::BM;
-    return ((N + 127) / 128) * ((M + bm - 1) / bm);
+struct W16Plan {
+    int tile;    // 0: 32 x 128, 1: 64 x 128, 2: 128 x 128, 3: 128 x 256
+    int splits;
+};
+
+// Up to 32 rows: the 32 x 128 tile, split along K to 512 workgroups.  Above: the tile and split
+// with the least predicted time.  A workgroup's step of two blocks takes, with 1, 2, 3 workgroups
+// on a CU (measured, us): 64 x 128 1.07, 1.86, 2.6; 128 x 128 1.7, 3.05; 128 x 256 2.85; a split
+// adds the reduction launch (2.5 us) and its traffic at 4 TB/s.  Splits only where the 128 x 128
+// grid leaves CUs idle, at least 4 steps each.  (Measured, us, best of all tiles and splits / this
+// rule's pick: 64 x 4096 x 4096 19.1 / 19.4; 128 x 14336 x 4096 58 / 58; 512 x 4096 x 4096 59.4 / 59.4;
+// 700 x 3008 x 3008 53.8 / 53.8; 1024 x 4096 x 4096 111 / 111; 218 x 2765 x 18176 92.7 / 95.)
+W16Plan w16_plan(int M, int N, int K) {
+    const int steps = K / 64;
+    const int grid128 = w16_tiles(M, N, 128, 128);
+    if (M <= kW16SmallRows) {
+        const int wgs = w16_tiles(M, N, kW16SmallRows, 128);
+        if (wgs >= kW16MinWGs) return {0, 1};
+        int sp = (kW16TargetWGs + wgs - 1) / wgs;
+        sp = sp < steps / 4 ? sp : steps / 4;
+        sp = sp < kW16MaxSplits ? sp : kW16MaxSplits;
+        return {0, sp < 1 ? 1 : sp};
+    }
+    constexpr int cap[4] = {0, 3, 2, 1};
+    constexpr double step_us[4][4] = {{}, {0.0, 1.07, 1.86, 2.6}, {0.0, 1.7, 3.05}, {0.0, 2.85}};
+    W16Plan best{1, 1};
+    double best_us = 1e30;
+    for (int tile = 1; tile <= 3; tile++) {
+        const int tiles = w16_tiles(M, N, tile == 1 ? 64 : 128, tile == 3 ? 256 : 128);
+        for (int sp = 1; sp <= kW16MaxSplits; sp++) {
+            if (sp > 1 && (grid128 >= kW16MinWGs || steps / sp < 4)) break;
+            const int per_cu = (int)(((long long)((tiles + 7) / 8) * sp + 31) / 32);   // on the fullest XCD
+            const double rounds = (double)(per_cu / cap[tile]) * step_us[tile][cap[tile]] + step_us[tile][per_cu % cap[tile]];
+            double us = rounds * ((steps + sp - 1) / sp);
+            if (sp > 1) us += 2.5 + (sp + 1) * (double)M * N * 4.0 / 4e6;
+            if (us < best_us) {
+                best_us = us;
+                best = {tile, sp};
+            }
+        }
+    }
+    return best;
 }
 }  // namespace
 
 int w16_splits(int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0 || w16_uses_gemv(M)) return 1;
-    const int wgs = w16_grid_wgs(M, N), steps = K / 64;
-    if (wgs >= kW16MinWGs) return 1;
-    int sp = (kW16TargetWGs + wgs - 1) / wgs;
-    sp = sp < steps / 4 ? sp : steps / 4;            // at least 4 K steps per split
-    sp = sp < kW16MaxSplits ? sp : kW16MaxSplits;
-    return sp < 1 ? 1 : sp;
+    return w16_plan(M, N, K).splits;
+}
+
+template <class T, int WT>
+static void w16_tile_launch(const float* A, const uint8_t* W, float* C, int M, int N, int nb, int splits, hipStream_t s) {
+    const int tiles = w16_tiles(M, N, T::BM, T::BN);
+    const dim3 grid((unsigned)((tiles + 7) / 8 * 8), 1u, (unsigned)splits);
+    hipLaunchKernelGGL((w16_kernel<T, WT>), grid, dim3(T::NT), 0, s, W, A, C, M, N, nb);
 }
 
 template <int WT>
-static hipError_t w16_launch(const float* A, const uint8_t* W, float* C, int M, int N, int K, int splits,
+static hipError_t w16_launch(const float* A, const uint8_t* W, float* C, int M, int N, int K, const W16Plan& p,
                              hipStream_t s) {
     const int nb = K / 32;
-    if (w16_skinny(M)) {
-        const dim3 grid((unsigned)((N + 127) / 128), (unsigned)((M + 31) / 32), (unsigned)splits);
-        hipLaunchKernelGGL((w16_kernel<W16Skinny, WT>), grid, dim3(256), 0, s, W, A, C, M, N, nb);
+    if (p.tile == 0) {
+        const dim3 grid((unsigned)((N + 127) / 128), (unsigned)((M + kW16SmallRows - 1) / kW16SmallRows), (unsigned)p.splits);
+        hipLaunchKernelGGL((w16_small_kernel<WT>), grid, dim3(256), 0, s, W, A, C, M, N, nb);
+    } else if (p.tile == 1) {
+        w16_tile_launch<W16Mid, WT>(A, W, C, M, N, nb, p.splits, s);
+    } else if (p.tile == 2) {
+        w16_tile_launch<W16Big, WT>(A, W, C, M, N, nb, p.splits, s);
     } else {
-        const int tiles = ((N + 127) / 128) * ((M + 127) / 128);
-        const dim3 grid((unsigned)((tiles + 7) / 8 * 8), 1u, (unsigned)splits);
-        hipLaunchKernelGGL((w16_kernel<W16Big, WT, true>), grid, dim3(256), 0, s, W, A, C, M, N, nb);
+        w16_tile_launch<W16Huge, WT>(A, W, C, M, N, nb, p.splits, s);
     }
     return hipGetLastError();
 }
@@ -482,15 +750,16 @@ hipError_t launch_w16(int wtype, const float* A, const uint8_t* W, float* C, int
         return wtype == kWQ40 ? w16_gemv_dispatch<kWQ40>(A, W, C, M, N, K, s)
                               : w16_gemv_dispatch<kWQ80>(A, W, C, M, N, K, s);
     }
-    const int splits = w16_splits(M, N, K);
+    const W16Plan plan = w16_plan(M, N, K);
+    const int splits = plan.splits;
     note_engine(KSQ_ENG_W16 | (splits > 1 ? KSQ_ENG_SPLITK : 0u));
     float* out = C;
     if (splits > 1) {
         if (!partials) return hipErrorInvalidValue;
         out = partials;
     }
-    hipError_t e = wtype == kWQ40 ? w16_launch<kWQ40>(A, W, out, M, N, K, splits, s)
-                                  : w16_launch<kWQ80>(A, W, out, M, N, K, splits, s);
+    hipError_t e = wtype == kWQ40 ? w16_launch<kWQ40>(A, W, out, M, N, K, plan, s)
+                                  : w16_launch<kWQ80>(A, W, out, M, N, K, plan, s);
     if (e != hipSuccess || splits == 1) return e;
     return launch_splitk_reduce(partials, C, (int64_t)M * N, splits, s);
 }

@@ -133,3 +133,37 @@ def test_w16_baseline_shapes(dev, oracle):
             rows = np.unique(np.linspace(0, M - 1, min(M, 8)).astype(int))
             ref = oracle.gemm_w16(wtype, x[rows], w, len(rows), N, K)
             assert _rel_err(y.cpu().numpy()[rows], ref) < TOL, (entry, M)
+
+
+# the 64 x 128, 128 x 128 and 128 x 256 tiles at their edges: one row past the small-batch form, rows and
+# columns one short of and one past a tile, one K step, an odd number of K steps, split along K
+@pytest.mark.parametrize("wtype", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(33, 1, 64), (64, 127, 128), (65, 129, 64), (33, 200, 1088), (257, 383, 192),
+                                   (1000, 4100, 128), (1025, 4097, 64), (2047, 4095, 64), (2048, 4097, 192)])
+def test_w16_tile_edges_exact(dev, wtype, M, N, K):
+    g = np.random.default_rng(900 + M + wtype)
+    w, vals = _int_weights(wtype, g, N, K)
+    amax = 250 if wtype == 0 else 15          # sum |a w| < 2^24, activations with two-term bf16 splits
+    x = g.integers(-amax, amax + 1, size=(M, K)).astype(np.float32)
+    want = x.astype(np.float64) @ vals.astype(np.float64).T
+    assert amax * (8 if wtype == 0 else 128) * K < 2 ** 24
+    y, eng = _run(dev, wtype, x, w, M, N, K, workspace=True)
+    assert np.array_equal(y, want.astype(np.float32)), (wtype, M, N, K, float(np.abs(y - want).max()))
+    assert "w16" in eng
+
+
+def test_w16_three_term_split(dev):
+    """Activations that need all 24 bits: a = 2^23 + odd integers against quants of -1, 0 and 1 (Q4_0
+    nibbles 7, 8, 9), one non-zero per row, so every output is one activation, exactly."""
+    M, N, K = 130, 300, 256
+    g = np.random.default_rng(77)
+    x = (g.integers(2 ** 23, 2 ** 24, size=(M, K)) | 1).astype(np.float32) * g.choice([-1.0, 1.0], size=(M, K)).astype(np.float32)
+    w = np.zeros((N, K // 32, 18), np.uint8)
+    w[..., 0:2] = np.frombuffer(np.float16(1).tobytes(), np.uint8)
+    w[..., 2:] = 0x88
+    pick = g.integers(0, K, size=N)
+    for n, k in enumerate(pick):
+        b, e = divmod(int(k), 32)
+        w[n, b, 2 + e % 16] = 0x89 if e < 16 else 0x98
+    y, _ = _run(dev, 0, x, w, M, N, K)
+    assert np.array_equal(y, x[:, pick])
