@@ -196,22 +196,29 @@ struct GemmWs {
     size_t q, p, total;
 };
 
-// Whether fp32 activations are quantised to planar block_q8_1 for the LDS-DMA GEMM (given that
-// the MFMA GEMM runs).
+// Whether fp32 activations are quantised to planar blocks for the LDS-DMA GEMM (given that the MFMA
+// GEMM runs).
 bool use_planar(int wtype, int atype, int M, int N, int K, bool mmq) {
-    return mmq && atype == KSQ_A_F32 && (K % 256) == 0 && ksq::mmq_planar_preferred(wtype, M, N, K);
+    return mmq && (atype == KSQ_A_F32 || (atype == KSQ_A_F32_Q8S && wtype == KSQ_W_Q8_0)) && (K % 256) == 0 &&
+           ksq::mmq_planar_preferred(wtype, M, N, K);
 }
 
-GemmWs gemm_ws(int wtype, int atype, int M, int N, int K, bool mmq) {
+// The planar form and the block form of one call differ in both parts (42 against 36 bytes per
+// block, and each tile's own split count), so the form is an argument.
+GemmWs gemm_ws(int wtype, int atype, int M, int N, int K, bool mmq, bool planar) {
     GemmWs w{};
-    w.q = use_planar(wtype, atype, M, N, K, mmq)
-              ? align256(ksq::planar_bytes(M, K))
-              : atype_raw(atype) ? align256((size_t)M * (size_t)(K / 32) * atype_block_bytes(atype)) : 0;
-    const int splits = mmq ? ksq::mmq_splits(wtype, M, N, K) : 1;
+    w.q = planar ? align256(ksq::planar_bytes(M, K))
+                 : atype_raw(atype) ? align256((size_t)M * (size_t)(K / 32) * atype_block_bytes(atype)) : 0;
+    const int splits = planar ? ksq::mmq_planar_splits(wtype, M, N, K) : mmq ? ksq::mmq_splits(wtype, M, N, K) : 1;
     w.p = splits > 1 ? align256((size_t)splits * (size_t)M * (size_t)N * sizeof(float)) : 0;
     w.total = w.q + w.p;
     return w;
 }
+
+// The byte-staged types (Q8_0, Q5_0, Q5_1) run in the planar form where its scratch is at hand and
+// in the block form where only that one's fits (a workspace, a pool under capture or the static
+// scratch of the smaller size).
+bool planar_optional(int wtype) { return wtype == KSQ_W_Q8_0 || wtype == KSQ_W_Q5_0 || wtype == KSQ_W_Q5_1; }
 
 int run_matmul(int wtype, int afmt, const uint8_t* W, const uint8_t* Aq, float* C, int M, int N, int K,
                float* partials, hipStream_t s) {
@@ -468,7 +475,7 @@ size_t ksq_gemm_workspace_size(int wtype, int atype, int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     const bool mmq_possible = atype_q8f(atype) ||
         ((g_path != 1) && (g_path == 2 || ksq::mmq_preferred(wtype, M, N, K)) && (K % 256) == 0);
-    return gemm_ws(wtype, atype, M, N, K, mmq_possible).total;
+    return gemm_ws(wtype, atype, M, N, K, mmq_possible, use_planar(wtype, atype, M, N, K, mmq_possible)).total;
 }
 
 int ksq_gemm(int wtype, int atype, const void* weight, const void* activation, float* output, int M, int N,
@@ -504,9 +511,14 @@ int ksq_gemm(int wtype, int atype, const void* weight, const void* activation, f
     // which is what the GEMM then reads
     const bool f32 = atype_f32(atype), f16 = atype == KSQ_A_F16;
     const bool mmq = atype_q8f(atype) || use_mmq(wtype, M, N, K, weight, f32 || f16 || aligned16(activation));
-    const GemmWs L = gemm_ws(wtype, atype, M, N, K, mmq);
+    bool planar = use_planar(wtype, atype, M, N, K, mmq);
+    GemmWs L = gemm_ws(wtype, atype, M, N, K, mmq, planar);
     uint8_t* ws = (uint8_t*)workspace;
     if (L.total) {
+        if (ws && planar && workspace_bytes < L.total && planar_optional(wtype)) {
+            planar = false;
+            L = gemm_ws(wtype, atype, M, N, K, mmq, false);
+        }
         if (ws) {
             if (workspace_bytes < L.total)
                 return set_error(KSQ_ERR_WORKSPACE, "workspace %zu < %zu bytes", workspace_bytes, L.total);
@@ -514,15 +526,20 @@ int ksq_gemm(int wtype, int atype, const void* weight, const void* activation, f
         } else {
             void* p = nullptr;
             st = pool_get(L.total, s, &p);
+            if (st == KSQ_ERR_WORKSPACE && planar && planar_optional(wtype)) {
+                planar = false;
+                L = gemm_ws(wtype, atype, M, N, K, mmq, false);
+                st = pool_get(L.total, s, &p);
+            }
             if (st != KSQ_OK) return st;
             ws = (uint8_t*)p;
         }
     }
     float* partials = L.p ? (float*)(ws + L.q) : nullptr;
-    if (use_planar(wtype, atype, M, N, K, mmq)) {
+    if (planar) {
         // the LDS-DMA GEMM's own activation layout (same blocks, split into planes)
         const ksq::PlanarQ81 P = ksq::planar_at(ws, M, K);
-        hipError_t e = ksq::launch_quantize_planar((const float*)activation, P, M, K, ksq::planar_da_scale(wtype), s);
+        hipError_t e = ksq::launch_quantize_planar(afmt, (const float*)activation, P, M, K, ksq::planar_da_scale(wtype), s);
         if (e != hipSuccess) return hip_error(e, "quantize launch");
         g_engines |= KSQ_ENG_QUANTIZE;
         e = ksq::launch_mmq_planar(wtype, (const uint8_t*)weight, P, output, M, N, K, partials, s);
@@ -551,8 +568,11 @@ int ksq_gemm_noalloc(int wtype, int atype, const void* weight, const void* activ
     int st = check_common(wtype, atype, weight, activation, output, M, N, K);
     if (st != KSQ_OK) return st;
     if (M == 0 || N == 0) return ok();
-    // the workspace ksq_gemm would ask for (an upper bound of what this call uses)
-    const size_t need = ksq_gemm_workspace_size(wtype, atype, M, N, K);
+    // the workspace ksq_gemm would ask for (an upper bound of what this call uses); the byte-staged
+    // types take the block form where the planar one does not fit
+    size_t need = ksq_gemm_workspace_size(wtype, atype, M, N, K);
+    if (need > (size_t)KSQ_NOALLOC_SCRATCH_BYTES && planar_optional(wtype) && use_planar(wtype, atype, M, N, K, true))
+        need = gemm_ws(wtype, atype, M, N, K, true, false).total;
     if (need > (size_t)KSQ_NOALLOC_SCRATCH_BYTES)
         return set_error(KSQ_ERR_WORKSPACE,
                          "ksq_gemm_noalloc: this call needs %zu bytes of scratch, more than the %u-byte static "
@@ -579,7 +599,7 @@ int ksq_debug_quantize_planar(int wtype, const float* x, void* planar, int M, in
     if (!x || !planar) return set_error(KSQ_ERR_NULL, "x or planar is NULL");
     if (((uintptr_t)x & 15u) || ((uintptr_t)planar & 255u))
         return set_error(KSQ_ERR_ALIGN, "x must be 16-byte and planar 256-byte aligned");
-    hipError_t e = ksq::launch_quantize_planar(x, ksq::planar_at(planar, M, K), M, K, ksq::planar_da_scale(wtype),
+    hipError_t e = ksq::launch_quantize_planar(ksq::kAQ81, x, ksq::planar_at(planar, M, K), M, K, ksq::planar_da_scale(wtype),
                                                (hipStream_t)stream);
     return e == hipSuccess ? ok() : hip_error(e, "quantize launch");
 }

@@ -47,14 +47,16 @@ struct PlanarQ81 {
 // Workspace bytes of the planes (each 256-byte aligned) and their addresses in a workspace.
 size_t planar_bytes(int M, int K);
 PlanarQ81 planar_at(void* ws, int M, int K);
-// fp32 [M][K] (16-byte aligned, K % 128 == 0) -> planar block_q8_1.
-hipError_t launch_quantize_planar(const float* x, const PlanarQ81& y, int M, int K, float da_scale, hipStream_t s);
+// fp32 [M][K] (16-byte aligned, K % 128 == 0) -> planar block_q8_1 (afmt kAQ81), or block_q8s (kAQ8S:
+// d with its two lowest mantissa bits cleared, sa zero).
+hipError_t launch_quantize_planar(int afmt, const float* x, const PlanarQ81& y, int M, int K, float da_scale,
+                                  hipStream_t s);
 // The same for the grouped MoE GEMM: x row m (m < T) goes to planar rows inv[m * top_k + s] (s <
 // top_k; -1: none); planar rows no entry maps to are not written.  With zero non-null the same
 // launch also clears nzero floats there (16-byte aligned, nzero % 4 == 0).
 hipError_t launch_quantize_planar_scatter(const float* x, const PlanarQ81& y, int T, int K, float da_scale,
                                           const int32_t* inv, int top_k, float* zero, int64_t nzero, hipStream_t s);
-// The LDS-DMA GEMM (Q4_0 / Q4_1 weights, K % 256 == 0, W 16-byte aligned) on planar
+// The LDS-DMA GEMM (32-element weight types, K % 256 == 0, W 16-byte aligned) on planar
 // activations quantised with da_scale = planar_da_scale(wtype); whether it is the pick for this
 // shape (fp32 activations); partials as launch_mmq (mmq_splits(...) > 1).
 bool mmq_planar_preferred(int wtype, int M, int N, int K);

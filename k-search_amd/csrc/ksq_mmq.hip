@@ -793,7 +793,7 @@ __global__ __launch_bounds__(T::NT, T::OCC) void mmq_kernel(const uint8_t* __res
     }
 }
 
-// ---- the LDS-DMA GEMM: planar block_q8_1 activations, nibble weights --------------------------
+// ---- the LDS-DMA GEMM: planar block_q8_1 activations ---------------------------------------------
 // 16 bytes per lane from global memory straight into LDS at lds + 16 * lane (no VGPRs); the
 // caller waits with s_waitcnt vmcnt before the data is read.
 __device__ __forceinline__ void dma16(const void* src, void* lds) {
@@ -802,7 +802,7 @@ __device__ __forceinline__ void dma16(const void* src, void* lds) {
 }
 __device__ __forceinline__ void wait_vmem_all() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-// 128 x 128 tiles of Q4_0 / Q4_1 weights against planar block_q8_1 activations, the same
+// 128 x 128 tiles of the 32-element weight types against planar block_q8_1 activations, the same
 // arithmetic as mmq_kernel (magic-bias epilogue, f16-MFMA side term) in K steps of 4 blocks
 // with every LDS array double-buffered, so the loads of step k+1 run under the MFMAs of step k:
 //  * every wave copies its share of step k+1's activation planes into the other buffer by DMA
@@ -821,6 +821,14 @@ __device__ __forceinline__ void wait_vmem_all() { asm volatile("s_waitcnt vmcnt(
 // 16 different bank groups (the plain p ^ (r % 8) left 2-way conflicts: 5.5e6 conflict cycles
 // per launch).  The slots of one DMA instruction are 8 consecutive rows, so lane l of
 // instruction i sources piece (l % 8) ^ ((4 i + l / 16) % 8).
+// Byte-staged weights (Q8_0; Q5_0 / Q5_1 widened while staging) lie in LDS as the activations do (128-byte
+// rows, swizzled pieces), so a fragment needs no unpacking.  Without the unpack between the reads
+// and the MFMAs the compiler ran a step's MFMAs ahead of their epilogues and its FMAs behind them
+// (600 registers spilled); empty asm statements on the fragments and on each sub-tile's accumulators
+// hold them to their region: no spill, Q8_0 M = 2048, N = K = 4096 95 us, M = 512, N = 14336, K = 4096 97
+// (GEMM alone; register-staged 128 x 128 tile 110).
+// Bound (Q4_0 M = 2048, N = K = 4096, timing-only variants on one box, GEMM 88.5 us): the vector pipe and
+// the MFMAs alone 69, their LDS reads 5, the global loads 10; without the MFMAs 78.
 // MOE (the expert-grouped GEMM): workgroup y is entry y of the tile schedule (128-row tiles of one
 // expert; surplus workgroups of the worst-case grid return at once).  Its planar rows are the
 // tile's rows of the expert-sorted entries (the gathered planar quantiser wrote them), the weights
@@ -831,18 +839,21 @@ __device__ __forceinline__ void wait_vmem_all() { asm volatile("s_waitcnt vmcnt(
 template <int WT, bool MOE = false>
 __global__ __launch_bounds__(256, 2) void mmq_planar_kernel(const uint8_t* __restrict__ W, PlanarQ81 A,
                                                            float* __restrict__ C, int M, int N, int nb, MoeTiles moe) {
-    static_assert(WT == kWQ40 || WT == kWQ41, "nibble-staged weights");
+    static_assert(!is_kquant(WT), "32-element block types");
     constexpr int KB = 4, BM = 128, BN = 128, TM = 4;
     using S = WShape<WT, KB>;
+    constexpr bool BYTES = !S::nib;     // int8 weight rows (Q5_0 / Q5_1 widened while staging)
+    constexpr bool SIDE = S::side;
+    constexpr int WP = BYTES ? 128 : S::WPitch;   // bytes of a staged weight row
     constexpr int WNW = S::Chunk / 4;   // weight words per row and step
     __shared__ __attribute__((aligned(16))) uint8_t sA0[BM * 128], sA1[BM * 128];
-    __shared__ __attribute__((aligned(16))) uint8_t sW0[BN * S::WPitch], sW1[BN * S::WPitch];
+    __shared__ __attribute__((aligned(16))) uint8_t sW0[BN * WP], sW1[BN * WP];
     __shared__ __attribute__((aligned(16))) float sDn0[KB * BM * 2], sDn1[KB * BM * 2];   // (d, nc) pairs
     __shared__ __attribute__((aligned(16))) float sDw0[KB * BN], sDw1[KB * BN];
-    __shared__ __attribute__((aligned(16))) uint16_t sSa0[BM * 4], sSa1[BM * 4];
-    // side-term weight factor per row and block; row BN stays zero (read by the lanes holding
-    // the f16 MFMA's k = 4..7, for which a step has no blocks)
-    __shared__ __attribute__((aligned(16))) uint16_t sDh0[(BN + 1) * 4], sDh1[(BN + 1) * 4];
+    __shared__ __attribute__((aligned(16))) uint16_t sSa0[SIDE ? BM * 4 : 8], sSa1[SIDE ? BM * 4 : 8];
+    // side-term weight factor per row and block (the lanes holding the f16 MFMA's k = 4..7, for
+    // which a step has no blocks, take zeros)
+    __shared__ __attribute__((aligned(16))) uint16_t sDh0[SIDE ? BN * 4 : 8], sDh1[SIDE ? BN * 4 : 8];
 
     __shared__ int32_t sRows[MOE ? BM : 1];   // MoE: entry index of each tile row
     __shared__ int32_t sTok[MOE ? BM : 1];    // MoE: its token (output row)
@@ -908,7 +919,7 @@ __global__ __launch_bounds__(256, 2) void mmq_planar_kernel(const uint8_t* __res
             for (int ii = 0; ii < 4; ii++) dma16(qs + qoff[ii], dA + (4 * wave + ii) * 1024);
         }
         dma16(A.dn + 2 * ((size_t)(kb0 + wave) * A.mp + m0 + 2 * lane), (P ? sDn1 : sDn0) + 256 * wave);
-        if (wave == 3) dma16(A.sa + ((size_t)(kb0 >> 2) * A.mp + m0 + 2 * lane) * 4, P ? sSa1 : sSa0);
+        if (SIDE && wave == 3) dma16(A.sa + ((size_t)(kb0 >> 2) * A.mp + m0 + 2 * lane) * 4, P ? sSa1 : sSa0);
     };
 
     // ---- weights: thread t stages blocks 2h, 2h + 1 (h = t / 128) of row t % 128 ----
@@ -937,13 +948,36 @@ __global__ __launch_bounds__(256, 2) void mmq_planar_kernel(const uint8_t* __res
             const int kb = 2 * wh + j, off = j * S::BB;
             const uint32_t dwb = half_at(pre, off);
             dDw[kb * BN + wsr] = f16_to_f32(dwb);
-            // side factor against -s_a: d_w (Q4_0) or -m (Q4_1)
-            dh[j] = (WT == kWQ41) ? (half_at(pre, off + 2) ^ 0x8000u) : dwb;
-            constexpr int q = (WT == kWQ40) ? 2 : 4;   // offset of qs
-            *(u32x4*)(dW + wsr * S::WPitch + kb * 16) =
-                u32x4{word_at(pre, off + q), word_at(pre, off + q + 4), word_at(pre, off + q + 8),
-                      word_at(pre, off + q + 12)};
+            // side factor against -s_a: d_w (Q4_0, Q5_0) or -m (Q4_1, Q5_1)
+            dh[j] = (WT == kWQ41 || WT == kWQ51) ? (half_at(pre, off + 2) ^ 0x8000u) : dwb;
+            if constexpr (!BYTES) {
+                constexpr int q = (WT == kWQ40) ? 2 : 4;   // offset of qs
+                *(u32x4*)(dW + wsr * WP + kb * 16) =
+                    u32x4{word_at(pre, off + q), word_at(pre, off + q + 4), word_at(pre, off + q + 8),
+                          word_at(pre, off + q + 12)};
+            } else {
+                // pieces 2 kb, 2 kb + 1 of the row, swizzled as the activation rows
+                const int sw = (wsr >> 1) & 7;
+                uint32_t o[8];
+                if constexpr (WT == kWQ80) {
+#pragma unroll
+                    for (int i = 0; i < 8; i++) o[i] = word_at(pre, off + 2 + 4 * i);
+                } else {
+                    // Q5: one byte per quant (0..31), the fifth bits from qh
+                    constexpr int qh = (WT == kWQ50) ? 2 : 4, q = qh + 4;
+                    const uint32_t h = word_at(pre, off + qh);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const uint32_t w4 = word_at(pre, off + q + 4 * i);
+                        o[i] = (w4 & 0x0F0F0F0Fu) | qh_to_bit4(h >> (4 * i));
+                        o[4 + i] = ((w4 >> 4) & 0x0F0F0F0Fu) | qh_to_bit4(h >> (16 + 4 * i));
+                    }
+                }
+                *(u32x4*)(dW + wsr * WP + (((2 * kb) ^ sw) << 4)) = u32x4{o[0], o[1], o[2], o[3]};
+                *(u32x4*)(dW + wsr * WP + (((2 * kb + 1) ^ sw) << 4)) = u32x4{o[4], o[5], o[6], o[7]};
+            }
         }
+        if constexpr (SIDE)
         *(uint32_t*)(dDh + 4 * wsr + 2 * wh) = dh[0] | (dh[1] << 16);
     };
 
@@ -960,8 +994,11 @@ __global__ __launch_bounds__(256, 2) void mmq_planar_kernel(const uint8_t* __res
     int aoff[KB];          // swizzled byte offset of piece 2b + hi of row l32
 #pragma unroll
     for (int b = 0; b < KB; b++) aoff[b] = l32 * 128 + (((2 * b + hi) ^ ((l32 >> 1) & 7)) << 4);
-    const int woff = (wn * 32 + l32) * S::WPitch;
-    const int dh_idx = hi ? BN * 4 : (wn * 32 + l32) * 4;
+    // this lane's weight piece of block b: 16 packed bytes (nibbles, unpacked per fragment) or the
+    // 16 int8 of its half
+    auto woff = [&](int b) __attribute__((always_inline)) -> int {
+        return BYTES ? wn * 32 * 128 + aoff[b] : (wn * 32 + l32) * WP + b * 16;
+    };
     const int nbase = wn * 32 + 4 * hi;   // local weight row of r = 0
 
     // TA: the row sub-tiles a K loop computes (TM, or fewer for a ragged MoE tile; each value
@@ -981,6 +1018,7 @@ __global__ __launch_bounds__(256, 2) void mmq_planar_kernel(const uint8_t* __res
         u32x4 bxn;
         f32x4 edw[4];
         auto unpack = [&](const u32x4& x) -> i32x4 {
+            if constexpr (BYTES) return __builtin_bit_cast(i32x4, x);
             const int s4 = 4 * hi;
             return i32x4{(int)((x.x >> s4) & 0x0F0F0F0Fu), (int)((x.y >> s4) & 0x0F0F0F0Fu),
                          (int)((x.z >> s4) & 0x0F0F0F0Fu), (int)((x.w >> s4) & 0x0F0F0F0Fu)};
@@ -988,9 +1026,9 @@ __global__ __launch_bounds__(256, 2) void mmq_planar_kernel(const uint8_t* __res
         if constexpr (TA >= 2) {
             // software pipeline, one region per MFMA q: issue the MFMA of q + 1, run the first
             // quarter of q's epilogue (its LDS operands were read during region q - 1), read the
-            // operands of q + 1 (its (d, nc) pair; at a block's first sub-tile the next block's
-            // fragments; a sub-tile before its last one the next block's weight scales), then the
-            // rest of q's epilogue.  The scheduling barriers hold that order: left to itself the
+            // operands of q + 1 (its (d, nc) pair; the next block's fragments into the registers
+            // whose last MFMA is issued; in a block's last region each quarter of the next block's
+            // weight scales as this block's is used up), then the rest of q's epilogue.  The scheduling barriers hold that order: left to itself the
             // compiler sank each MFMA to its first use and waited on the LDS reads it had just
             // issued (config 2, GEMM alone: 93.4 -> 91.5 us, MoE config 4: 264 -> 257, same bits).
             auto quarter = [&](const i32x16& c, auto iv, int qq, const f32x2& dn) __attribute__((always_inline)) {
@@ -1006,26 +1044,26 @@ __global__ __launch_bounds__(256, 2) void mmq_planar_kernel(const uint8_t* __res
 #pragma unroll
                 for (int p = 0; p < 4; p++) acc[i][4 * qq + p] = fmaf(edw[qq][p], x[p], acc[i][4 * qq + p]);
             };
-            f32x4 edwn[4];
             f32x2 dnc = *(const f32x2*)&cDn[2 * l32];
 #pragma unroll
             for (int qq = 0; qq < 4; qq++) edw[qq] = *(const f32x4*)&cDw[nbase + 8 * qq];
 #pragma unroll
             for (int ii = 0; ii < TA; ii++) af[ii] = *(const i32x4*)(cA + ii * 32 * 128 + aoff[0]);
-            bf = unpack(*(const u32x4*)(cW + woff));
+            bf = unpack(*(const u32x4*)(cW + woff(0)));
             __builtin_amdgcn_s_setprio(2);
             i32x16 cur = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf, af[0], bias, 0, 0, 0);
+            asm volatile("" : "+v"(cur));
             static_for<NQ>([&](auto qv) __attribute__((always_inline)) {
                 constexpr int q = decltype(qv)::value;
                 constexpr int b = q / TA, i = q % TA;
                 i32x16 nxt = bias;
                 if constexpr (q + 1 < NQ) {
                     if constexpr (i + 1 < TA) {
+                        if constexpr (BYTES) asm volatile("" : "+v"(af[i + 1]));
                         nxt = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf, af[i + 1], bias, 0, 0, 0);
                     } else {
                         bf = unpack(bxn);
-#pragma unroll
-                        for (int ii = 0; ii < TA; ii++) af[ii] = afn[ii];
+                        if constexpr (BYTES) asm volatile("" : "+v"(bf), "+v"(af[0]));
                         nxt = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf, af[0], bias, 0, 0, 0);
                     }
                     asm volatile("" : "+v"(nxt));   // pins the issue here, ahead of q's epilogue
@@ -1038,29 +1076,28 @@ __global__ __launch_bounds__(256, 2) void mmq_planar_kernel(const uint8_t* __res
                     constexpr int bn = (q + 1) / TA, in = (q + 1) % TA;
                     dnn = *(const f32x2*)&cDn[2 * (bn * BM + in * 32 + l32)];
                 }
-                if constexpr (i == 0 && b + 1 < KB) {
-#pragma unroll
-                    for (int ii = 0; ii < TA; ii++) afn[ii] = *(const i32x4*)(cA + ii * 32 * 128 + aoff[b + 1]);
-                    bxn = *(const u32x4*)(cW + woff + (b + 1) * 16);
+                if constexpr (b + 1 < KB && i < TA - 1) {
+                    // the fragments whose last MFMA is issued: the next block's into their registers
+                    if constexpr (i == 0) af[0] = *(const i32x4*)(cA + aoff[b + 1]);
+                    af[i + 1] = *(const i32x4*)(cA + (i + 1) * 32 * 128 + aoff[b + 1]);
+                    if constexpr (i == TA - 2) bxn = *(const u32x4*)(cW + woff(b + 1));
                 }
-                if constexpr (i == TA - 2 && b + 1 < KB) {
-#pragma unroll
-                    for (int qq = 0; qq < 4; qq++) edwn[qq] = *(const f32x4*)&cDw[(b + 1) * BN + nbase + 8 * qq];
-                }
+                if constexpr (i == TA - 1 && b + 1 < KB) edw[0] = *(const f32x4*)&cDw[(b + 1) * BN + nbase];
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int qq = 1; qq < 4; qq++) quarter(cur, IntC<i>{}, qq, dnc);
-                if constexpr (i == TA - 1 && b + 1 < KB) {
-#pragma unroll
-                    for (int qq = 0; qq < 4; qq++) edw[qq] = edwn[qq];
+                for (int qq = 1; qq < 4; qq++) {
+                    quarter(cur, IntC<i>{}, qq, dnc);
+                    if constexpr (i == TA - 1 && b + 1 < KB) edw[qq] = *(const f32x4*)&cDw[(b + 1) * BN + nbase + 8 * qq];
                 }
+                if constexpr (BYTES) asm volatile("" : "+v"(acc[i]));
+                __builtin_amdgcn_sched_barrier(0);
                 dnc = dnn;
                 cur = nxt;
             });
         } else {
     #pragma unroll
             for (int ii = 0; ii < TA; ii++) af[ii] = *(const i32x4*)(cA + ii * 32 * 128 + aoff[0]);
-            bf = unpack(*(const u32x4*)(cW + woff));
+            bf = unpack(*(const u32x4*)(cW + woff(0)));
             __builtin_amdgcn_s_setprio(2);
             i32x16 cur = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf, af[0], bias, 0, 0, 0);
     #pragma unroll
@@ -1070,7 +1107,7 @@ __global__ __launch_bounds__(256, 2) void mmq_planar_kernel(const uint8_t* __res
                     // the next block's fragments, a block ahead of their MFMAs
     #pragma unroll
                     for (int ii = 0; ii < TA; ii++) afn[ii] = *(const i32x4*)(cA + ii * 32 * 128 + aoff[b + 1]);
-                    bxn = *(const u32x4*)(cW + woff + (b + 1) * 16);
+                    bxn = *(const u32x4*)(cW + woff(b + 1));
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 i32x16 nxt = bias;
@@ -1108,19 +1145,18 @@ __global__ __launch_bounds__(256, 2) void mmq_planar_kernel(const uint8_t* __res
         }
         __builtin_amdgcn_s_setprio(0);
         // side term over the step's 4 blocks (f16 MFMA, exact products; k = 4..7 read zeros)
-        const f16x4 dw4 = *(const f16x4*)&cDh[dh_idx];
+        if constexpr (SIDE) {
+            const u32x2 dwv = *(const u32x2*)&cDh[(wn * 32 + l32) * 4];
+            const f16x4 dw4 = __builtin_bit_cast(f16x4, u32x2{hi ? 0u : dwv.x, hi ? 0u : dwv.y});
 #pragma unroll
-        for (int i = 0; i < TA; i++) {
-            const f16x4 sa4 = *(const f16x4*)&cSa[(i * 32 + l32) * 4];
-            acc[i] = __builtin_amdgcn_mfma_f32_32x32x8f16(dw4, sa4, acc[i], 0, 0, 0);
+            for (int i = 0; i < TA; i++) {
+                const f16x4 sa4 = *(const f16x4*)&cSa[(i * 32 + l32) * 4];
+                acc[i] = __builtin_amdgcn_mfma_f32_32x32x8f16(dw4, sa4, acc[i], 0, 0, 0);
+            }
         }
     };
 
     // ---- pipeline ----
-    if (t < 4) {
-        sDh0[BN * 4 + t] = 0;
-        sDh1[BN * 4 + t] = 0;
-    }
     auto run = [&](auto tav) __attribute__((always_inline)) {
         constexpr int TA = decltype(tav)::value;
         // waves past the computed sub-tiles stage no activation quants (no wave reads them)
@@ -1503,20 +1539,30 @@ hipError_t launch_mmq(int wtype, int afmt, const uint8_t* W, const uint8_t* A, f
     return launch_splitk_reduce(partials, C, (int64_t)M * N, splits, s);
 }
 
-// The LDS-DMA GEMM takes fp32 activations against Q4_0 / Q4_1 wherever the 128 x 128 tile is
-// the automatic pick (or configuration 8 forces it).
+// The LDS-DMA GEMM takes fp32 activations (block_q8_1, and block_q8s for Q8_0) against the nibble
+// types wherever the 128 x 128 tile is the automatic pick, and against the byte-staged types from a
+// 128 x 128 grid of 300 workgroups on (whole call, us, the register-staged pick vs this kernel: Q8_0
+// M = 2048, N = K = 4096 (512 workgroups) 137 vs 120, M = 512, N = 14336, K = 4096 (448) 121 vs 106,
+// M = 1000, N = 5000, K = 4096 (320) 110 vs 93, M = 2043, N = 9088, K = 1024 98 vs 83; at 256 and 224
+// workgroups level: 75.4 vs 75.9, 110 vs 114; below behind: M = 256, N = 14336 68 vs 77).
+// Configuration 8 forces it.
 #ifndef KSQ_MMQ_PLANAR
 #define KSQ_MMQ_PLANAR 1
 #endif
+constexpr int kPlanarByteMinWGs = 300;
 bool mmq_planar_preferred(int wtype, int M, int N, int K) {
-    if (wtype != kWQ40 && wtype != kWQ41) return false;
+    if (is_kquant(wtype)) return false;
     if (g_mmq_config == 8) return true;
-    return KSQ_MMQ_PLANAR && g_mmq_config == 0 && pick_config(wtype, M, N, K) == 1;
+    if (!KSQ_MMQ_PLANAR || g_mmq_config != 0) return false;
+    if (wtype == kWQ40 || wtype == kWQ41) return pick_config(wtype, M, N, K) == 1;
+    return grid_wgs<TileL>(M, N) >= kPlanarByteMinWGs;
 }
 
 int mmq_planar_splits(int wtype, int M, int N, int K) { return split_for<TileL>(wtype, M, N, K); }
 
-float planar_da_scale(int wtype) { return wtype == kWQ40 ? 1.0f / WShape<kWQ40, 4>::out_scale : 1.0f; }
+float planar_da_scale(int wtype) {
+    return wtype == kWQ40 ? 1.0f / WShape<kWQ40, 4>::out_scale : wtype == kWQ50 ? 1.0f / WShape<kWQ50, 4>::out_scale : 1.0f;
+}
 
 hipError_t launch_mmq_planar(int wtype, const uint8_t* W, const PlanarQ81& A, float* C, int M, int N, int K,
                              float* partials, hipStream_t s) {
@@ -1527,12 +1573,17 @@ hipError_t launch_mmq_planar(int wtype, const uint8_t* W, const PlanarQ81& A, fl
     const int tiles = ((N + 127) / 128) * ((M + 127) / 128);
     const dim3 grid((unsigned)((tiles + 7) / 8 * 8), 1u, (unsigned)splits);   // tile order: xcd_tile
     float* out = splits > 1 ? partials : C;
-    if (wtype == kWQ40)
-        hipLaunchKernelGGL((mmq_planar_kernel<kWQ40, false>), grid, dim3(256), 0, s, W, A, out, M, N, K / 32, MoeTiles{});
-    else if (wtype == kWQ41)
-        hipLaunchKernelGGL((mmq_planar_kernel<kWQ41, false>), grid, dim3(256), 0, s, W, A, out, M, N, K / 32, MoeTiles{});
-    else
-        return hipErrorNotSupported;
+#define KSQ_PLANAR_CASE(WT) \
+    case WT: hipLaunchKernelGGL((mmq_planar_kernel<WT, false>), grid, dim3(256), 0, s, W, A, out, M, N, K / 32, MoeTiles{}); break;
+    switch (wtype) {
+        KSQ_PLANAR_CASE(kWQ40)
+        KSQ_PLANAR_CASE(kWQ41)
+        KSQ_PLANAR_CASE(kWQ80)
+        KSQ_PLANAR_CASE(kWQ50)
+        KSQ_PLANAR_CASE(kWQ51)
+        default: return hipErrorNotSupported;
+    }
+#undef KSQ_PLANAR_CASE
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || splits == 1) return e;
     return launch_splitk_reduce(partials, C, (int64_t)M * N, splits, s);

@@ -185,7 +185,9 @@ hipError_t launch_quantize_q8_1_zero(const float* x, uint8_t* y, int64_t rows, i
 // R rows per workgroup (4 R threads, each loading 8 16-byte pieces): the dense form takes 16 rows
 // (8 KiB per workgroup, the read curve's best shape at this size): 10.47 -> 10.00 us at config 2
 // against 64 rows, three trace pairs.
-template <bool SCATTER, int R = 64>
+// Q8S: by the native W8A8C8 operator's rules (block_q8s: fp32 d, its two lowest mantissa bits cleared so
+// that 12582912 * d stays exact; no sum).
+template <bool SCATTER, int R = 64, bool Q8S = false>
 __global__ __launch_bounds__(4 * R) void quantize_planar_kernel(const float* __restrict__ x, PlanarQ81 y, int M, int K,
                                                               float da_scale, const int32_t* __restrict__ inv,
                                                               int top_k, float* __restrict__ zero, int64_t n4) {
@@ -225,9 +227,10 @@ __global__ __launch_bounds__(4 * R) void quantize_planar_kernel(const float* __r
 #pragma unroll
     for (int j = 0; j < 32; j++) v[j] = stage[t * kQPitch + j];
     uint32_t q[9];
-    quantize_block_q8_1(v, q);
-    const float d = f16_to_f32(q[0] & 0xFFFFu) * da_scale;
-    const uint16_t sa = (uint16_t)((q[0] >> 16) ^ 0x8000u);
+    if constexpr (Q8S) quantize_block_q8s(v, q);
+    else quantize_block_q8_1(v, q);
+    const float d = (Q8S ? __builtin_bit_cast(float, q[0] & ~3u) : f16_to_f32(q[0] & 0xFFFFu)) * da_scale;
+    const uint16_t sa = Q8S ? (uint16_t)0 : (uint16_t)((q[0] >> 16) ^ 0x8000u);
     auto put = [&](int pm, bool quants) __attribute__((always_inline)) {
         if (quants) {
             u32x4* dq = (u32x4*)(y.q + (size_t)pm * K + (size_t)kb * 32);
@@ -268,13 +271,18 @@ PlanarQ81 planar_at(void* ws, int M, int K) {
     return y;
 }
 
-hipError_t launch_quantize_planar(const float* x, const PlanarQ81& y, int M, int K, float da_scale, hipStream_t s) {
+hipError_t launch_quantize_planar(int afmt, const float* x, const PlanarQ81& y, int M, int K, float da_scale,
+                                  hipStream_t s) {
     if (M <= 0 || K <= 0) return hipSuccess;
     if (K % 128) return hipErrorInvalidValue;
     constexpr int R = 16;
     const dim3 grid((unsigned)(y.mp / R), (unsigned)(K / 128));
-    hipLaunchKernelGGL((quantize_planar_kernel<false, R>), grid, dim3(4 * R), 0, s, x, y, M, K, da_scale, nullptr, 1,
-                       nullptr, (int64_t)0);
+    if (afmt == kAQ8S)
+        hipLaunchKernelGGL((quantize_planar_kernel<false, R, true>), grid, dim3(4 * R), 0, s, x, y, M, K, da_scale,
+                           nullptr, 1, nullptr, (int64_t)0);
+    else
+        hipLaunchKernelGGL((quantize_planar_kernel<false, R>), grid, dim3(4 * R), 0, s, x, y, M, K, da_scale, nullptr,
+                           1, nullptr, (int64_t)0);
     return hipGetLastError();
 }
 

@@ -240,6 +240,16 @@ def _engine_cases():
         # a single row and a ragged 33 rows in one 128-row tile (rows past M read row M-1)
         for M in (1, 33):
             cases.append((f"mmqp_m{M}_w{wt}", wt, M, 136, 512, 0, 2, 8, {"quantize", "mmq_planar"}, 0))
+    # the same kernel on the byte-staged types (its own grid order: split and unsplit, odd and even
+    # steps, ragged rows), and with block_q8s activations
+    for wt in (1, 5, 6):
+        for M, N, K, sp in ((200, 330, 1024, True), (200, 330, 1280, True), (1, 136, 512, False), (33, 136, 512, False),
+                            (129, 129, 256, False)):
+            cases.append((f"mmqp_m{M}_k{K}_w{wt}", wt, M, N, K, 0, 2, 8, {"quantize", "mmq_planar"} | ({"splitk"} if sp else set()), 0))
+    cases.append(("mmqp_q8s", 1, 140, 200, 768, 2, 2, 8, {"quantize", "mmq_planar"}, 0))
+    # the automatic route at its first grid (300 workgroups of 128 x 128)
+    for wt in (1, 5, 6):
+        cases.append((f"mmqp_auto_w{wt}", wt, 1500, 3100, 256, 0, 0, 0, {"quantize", "mmq_planar"}, 0))
     cases.append(("splitk_w0", 0, 32, 1024, 8192, 1, 2, 0, {"mmq5", "splitk"}, 0))
     cases.append(("splitk_w1", 1, 32, 1024, 8192, 1, 2, 0, {"mmq3", "splitk"}, 0))
     # the native W8A8C8 operator's block_q8s activations: fp32 (its quantiser) and pre-quantised
@@ -476,3 +486,29 @@ def test_dropin_forwarding_module(dev):
         assert st == 0, entry
         assert np.array_equal(y.cpu().numpy(), _exact(wtype, blocks, w, q8s=atype == 2)), entry
     assert D.dropin_forward(b"no_such_entry", None, None, None, 1, 1, 32) == -1
+
+
+@pytest.mark.parametrize("wtype", [1, 5, 6])
+def test_byte_types_block_form_workspace(dev, wtype):
+    """A large fp32 call of the byte-staged types with a workspace of the block form's size (36 bytes
+    per activation block), smaller than the planar form's, runs in the block form, exactly; with
+    one byte less it is refused."""
+    import torch
+    from ksq import _lib, ops, refcheck
+    from oracle import oracle
+    M, N, K = 1500, 3100, 256
+    g = np.random.default_rng(4700 + wtype)
+    w = refcheck.unit_weights(wtype, g, N, K)
+    x = refcheck.unit_activations(g, M, K, qmax=QMAX_F32[wtype], onehot=refcheck.onehot_pattern(M, K // 32))
+    need = (M * (K // 32) * 36 + 255) // 256 * 256
+    assert ops.workspace_size(wtype, 0, M, N, K) > need
+    ws = torch.empty(need, dtype=torch.uint8, device=dev)
+    y = ops.gemm(wtype, 0, _t(w, dev), _t(x, dev), M, N, K, workspace=ws)
+    eng = ops.last_engines()
+    torch.cuda.synchronize()
+    assert "mmq_planar" not in eng and "quantize" in eng, eng
+    cols = np.arange(0, N, 97)
+    ref = oracle.gemm_f64(wtype, oracle.quantize_q8_1(x), w[cols], M, len(cols), K)
+    assert np.array_equal(y.cpu().numpy()[:, cols], ref.astype(np.float32))
+    with pytest.raises(_lib.KsqError):
+        ops.gemm(wtype, 0, _t(w, dev), _t(x, dev), M, N, K, workspace=ws[:need - 1])
