@@ -521,10 +521,12 @@ __device__ __forceinline__ float reg_block_dot_q8f(const uint32_t* raw, const ui
 
 // C[m][row] for m < MR (1 or 2); RPW rows per 256-thread workgroup: 8 = two rows per wave (each
 // activation pair a lane loads serves both), 4 = one, 2 or 1 = 4 / RPW waves per row (their
-// partial sums meet in LDS).  A: block_q8_1 (or block_q8s when AS) [MR][nb], nb even.
+// partial sums meet in LDS).  A: block_q8_1 (or block_q8s when AS) [MR][nb], nb even.  Output
+// C[m * ldc + row * ldr].
 template <int WT, int MR, bool AS, int RPW>
 __global__ __launch_bounds__(256) void gemv_direct_kernel(const uint8_t* __restrict__ W, const uint8_t* __restrict__ A,
-                                                          float* __restrict__ C, int N, int nb, int ldc) {
+                                                          float* __restrict__ C, int N, int nb, int ldc,
+                                                          int ldr) {
     static_assert(!is_kquant(WT) && (MR == 1 || MR == 2), "32-element block types, 1-2 activation rows");
     constexpr int WPR = RPW >= 4 ? 1 : 4 / RPW;  // waves per row
     constexpr int VR = RPW >= 4 ? RPW / 4 : 1;   // rows per wave
@@ -580,7 +582,7 @@ __global__ __launch_bounds__(256) void gemv_direct_kernel(const uint8_t* __restr
         for (int v = 0; v < VR; v++)
             if (row0 + v < N) {
 #pragma unroll
-                for (int m = 0; m < MR; m++) C[(size_t)m * ldc + row0 + v] = acc[v][m];
+                for (int m = 0; m < MR; m++) C[(size_t)m * ldc + (size_t)(row0 + v) * ldr] = acc[v][m];
             }
     }
 }
@@ -1152,13 +1154,13 @@ static int direct_rpw(int rpw, int N, int nb) {
 
 template <int WT, bool AS, int MR>
 static hipError_t direct_launch_rpw(int rpw, const uint8_t* W, const uint8_t* A, float* C, int N, int nb, int ldc,
-                                    hipStream_t s) {
+                                    int ldr, hipStream_t s) {
     const dim3 blk(256);
     switch (direct_rpw(rpw, N, nb)) {
-        case 8: hipLaunchKernelGGL((gemv_direct_kernel<WT, MR, AS, 8>), dim3((N + 7) / 8), blk, 0, s, W, A, C, N, nb, ldc); break;
-        case 4: hipLaunchKernelGGL((gemv_direct_kernel<WT, MR, AS, 4>), dim3((N + 3) / 4), blk, 0, s, W, A, C, N, nb, ldc); break;
-        case 2: hipLaunchKernelGGL((gemv_direct_kernel<WT, MR, AS, 2>), dim3((N + 1) / 2), blk, 0, s, W, A, C, N, nb, ldc); break;
-        default: hipLaunchKernelGGL((gemv_direct_kernel<WT, MR, AS, 1>), dim3(N), blk, 0, s, W, A, C, N, nb, ldc); break;
+        case 8: hipLaunchKernelGGL((gemv_direct_kernel<WT, MR, AS, 8>), dim3((N + 7) / 8), blk, 0, s, W, A, C, N, nb, ldc, ldr); break;
+        case 4: hipLaunchKernelGGL((gemv_direct_kernel<WT, MR, AS, 4>), dim3((N + 3) / 4), blk, 0, s, W, A, C, N, nb, ldc, ldr); break;
+        case 2: hipLaunchKernelGGL((gemv_direct_kernel<WT, MR, AS, 2>), dim3((N + 1) / 2), blk, 0, s, W, A, C, N, nb, ldc, ldr); break;
+        default: hipLaunchKernelGGL((gemv_direct_kernel<WT, MR, AS, 1>), dim3(N), blk, 0, s, W, A, C, N, nb, ldc, ldr); break;
     }
     return hipGetLastError();
 }
@@ -1195,8 +1197,8 @@ static hipError_t direct_launch(bool quant, bool xh, int mr, int rpw, const uint
                            : direct_fq_launch_rpw<WT, AS, 2, false>(rpw, W, A, C, N, nb, ldc, ldr, s);
         }
     }
-    return mr == 1 ? direct_launch_rpw<WT, AS, 1>(rpw, W, (const uint8_t*)A, C, N, nb, ldc, s)
-                   : direct_launch_rpw<WT, AS, 2>(rpw, W, (const uint8_t*)A, C, N, nb, ldc, s);
+    return mr == 1 ? direct_launch_rpw<WT, AS, 1>(rpw, W, (const uint8_t*)A, C, N, nb, ldc, ldr, s)
+                   : direct_launch_rpw<WT, AS, 2>(rpw, W, (const uint8_t*)A, C, N, nb, ldc, ldr, s);
 }
 
 // Pairs per K tile of gemv_direct_mr_kernel: the whole row while MR rows of it fit the LDS

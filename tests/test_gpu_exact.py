@@ -460,6 +460,22 @@ def test_fp16_fused_routes_exact(dev, Mw, Na, K, engines):
     assert eng == engines, eng
 
 
+@pytest.mark.parametrize("Mw,Na", [(13760, 2), (26880, 1), (26888, 2)])
+def test_fp16_fused_decode_past_work_limit(dev, Mw, Na):
+    """One and two activation rows past the in-workgroup quantisation's work limit: the register-direct
+    kernel on the quantised rows stores [N][M] results with their stride."""
+    import torch
+    from ksq import ops, refcheck
+    K = 4096
+    g = np.random.default_rng(4950 + Na)
+    w, xh, blocks = _inputs(0, g, Na, Mw, K, 4, refcheck.onehot_pattern(Na, K // 32))
+    y = ops.gemm_q4_0_fp16_fused(_t(w, dev), _t(xh, dev), Mw, Na, K)
+    eng = ops.last_engines()
+    torch.cuda.synchronize()
+    assert np.array_equal(y.cpu().numpy(), _exact(0, blocks, w).T)
+    assert eng == {"quantize", "gemv_direct"}, eng
+
+
 def test_dropin_forwarding_module(dev):
     """The forwarding kernel.cpp a maintainer compiles in place of a definition's kernel.cu
     (tests/dropin/kernel.cpp, built by __graft_entry__.build() with hipcc against include/ksq.h
