@@ -221,8 +221,8 @@ KSQ_API int ksq_gemm_w8a16(const float* A, const uint8_t* B, float* C, int M, in
 
 /* Workspace bytes ksq_gemm needs for (wtype, atype, M, N, K): the quantised copy of fp32 or
  * fp16 activations (block_q8_1 rows, or the LDS-DMA GEMM's planar form for fp32 activations
- * at large M, 42 bytes per block; Q8_0, Q5_0 and Q5_1 calls with a workspace of the block form's
- * size, 36 bytes per block, take that form instead), plus the split-K partial sums of small MFMA grids (so it can
+ * at large M, 42 bytes per block; for Q8_0, Q5_0 and Q5_1 the block form's 36 bytes, and a call
+ * whose workspace holds 42 takes the faster planar form), plus the split-K partial sums of small MFMA grids (so it can
  * be non-zero for pre-quantised activations too).  The workspace must be 16-byte aligned. */
 KSQ_API size_t ksq_gemm_workspace_size(int wtype, int atype, int M, int N, int K);
 

@@ -475,7 +475,10 @@ size_t ksq_gemm_workspace_size(int wtype, int atype, int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     const bool mmq_possible = atype_q8f(atype) ||
         ((g_path != 1) && (g_path == 2 || ksq::mmq_preferred(wtype, M, N, K)) && (K % 256) == 0);
-    return gemm_ws(wtype, atype, M, N, K, mmq_possible, use_planar(wtype, atype, M, N, K, mmq_possible)).total;
+    // the block form's size where the planar form is optional: a caller's workspace of that size is
+    // enough, a larger one that holds the planar form is used for it
+    const bool planar = !planar_optional(wtype) && use_planar(wtype, atype, M, N, K, mmq_possible);
+    return gemm_ws(wtype, atype, M, N, K, mmq_possible, planar).total;
 }
 
 int ksq_gemm(int wtype, int atype, const void* weight, const void* activation, float* output, int M, int N,
@@ -568,11 +571,8 @@ int ksq_gemm_noalloc(int wtype, int atype, const void* weight, const void* activ
     int st = check_common(wtype, atype, weight, activation, output, M, N, K);
     if (st != KSQ_OK) return st;
     if (M == 0 || N == 0) return ok();
-    // the workspace ksq_gemm would ask for (an upper bound of what this call uses); the byte-staged
-    // types take the block form where the planar one does not fit
-    size_t need = ksq_gemm_workspace_size(wtype, atype, M, N, K);
-    if (need > (size_t)KSQ_NOALLOC_SCRATCH_BYTES && planar_optional(wtype) && use_planar(wtype, atype, M, N, K, true))
-        need = gemm_ws(wtype, atype, M, N, K, true, false).total;
+    // the workspace ksq_gemm asks for; the byte-staged types take the planar form where it fits too
+    const size_t need = ksq_gemm_workspace_size(wtype, atype, M, N, K);
     if (need > (size_t)KSQ_NOALLOC_SCRATCH_BYTES)
         return set_error(KSQ_ERR_WORKSPACE,
                          "ksq_gemm_noalloc: this call needs %zu bytes of scratch, more than the %u-byte static "
