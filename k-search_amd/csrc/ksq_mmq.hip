@@ -851,9 +851,11 @@ __global__ __launch_bounds__(256, 2) void mmq_planar_kernel(const uint8_t* __res
     __shared__ __attribute__((aligned(16))) float sDn0[KB * BM * 2], sDn1[KB * BM * 2];   // (d, nc) pairs
     __shared__ __attribute__((aligned(16))) float sDw0[KB * BN], sDw1[KB * BN];
     __shared__ __attribute__((aligned(16))) uint16_t sSa0[SIDE ? BM * 4 : 8], sSa1[SIDE ? BM * 4 : 8];
-    // side-term weight factor per row and block (the lanes holding the f16 MFMA's k = 4..7, for
-    // which a step has no blocks, take zeros)
-    __shared__ __attribute__((aligned(16))) uint16_t sDh0[SIDE ? BN * 4 : 8], sDh1[SIDE ? BN * 4 : 8];
+    // side-term weight factor per row and block; the lanes holding the f16 MFMA's k = 4..7, for
+    // which a step has no blocks, read zeros: row BN, or (byte types, whose LDS is full) a select
+    constexpr bool ZROW = SIDE && !BYTES;
+    constexpr int DhN = SIDE ? (BN + (ZROW ? 1 : 0)) * 4 : 8;
+    __shared__ __attribute__((aligned(16))) uint16_t sDh0[DhN], sDh1[DhN];
 
     __shared__ int32_t sRows[MOE ? BM : 1];   // MoE: entry index of each tile row
     __shared__ int32_t sTok[MOE ? BM : 1];    // MoE: its token (output row)
@@ -977,8 +979,7 @@ __global__ __launch_bounds__(256, 2) void mmq_planar_kernel(const uint8_t* __res
                 *(u32x4*)(dW + wsr * WP + (((2 * kb + 1) ^ sw) << 4)) = u32x4{o[4], o[5], o[6], o[7]};
             }
         }
-        if constexpr (SIDE)
-        *(uint32_t*)(dDh + 4 * wsr + 2 * wh) = dh[0] | (dh[1] << 16);
+        if constexpr (SIDE) *(uint32_t*)(dDh + 4 * wsr + 2 * wh) = dh[0] | (dh[1] << 16);
     };
 
     // ---- compute ----
@@ -999,6 +1000,7 @@ __global__ __launch_bounds__(256, 2) void mmq_planar_kernel(const uint8_t* __res
     auto woff = [&](int b) __attribute__((always_inline)) -> int {
         return BYTES ? wn * 32 * 128 + aoff[b] : (wn * 32 + l32) * WP + b * 16;
     };
+    const int dh_idx = (ZROW && hi) ? BN * 4 : (wn * 32 + l32) * 4;
     const int nbase = wn * 32 + 4 * hi;   // local weight row of r = 0
 
     // TA: the row sub-tiles a K loop computes (TM, or fewer for a ragged MoE tile; each value
@@ -1026,11 +1028,17 @@ __global__ __launch_bounds__(256, 2) void mmq_planar_kernel(const uint8_t* __res
         if constexpr (TA >= 2) {
             // software pipeline, one region per MFMA q: issue the MFMA of q + 1, run the first
             // quarter of q's epilogue (its LDS operands were read during region q - 1), read the
-            // operands of q + 1 (its (d, nc) pair; the next block's fragments into the registers
-            // whose last MFMA is issued; in a block's last region each quarter of the next block's
-            // weight scales as this block's is used up), then the rest of q's epilogue.  The scheduling barriers hold that order: left to itself the
+            // operands of q + 1 (its (d, nc) pair; at a block's first sub-tile the next block's
+            // fragments; a sub-tile before its last one the next block's weight scales), then the
+            // rest of q's epilogue.  The scheduling barriers hold that order: left to itself the
             // compiler sank each MFMA to its first use and waited on the LDS reads it had just
             // issued (config 2, GEMM alone: 93.4 -> 91.5 us, MoE config 4: 264 -> 257, same bits).
+            // Byte-staged weights need the registers: the next block's fragments go into those
+            // whose last MFMA is issued, and in a block's last region each quarter of its weight
+            // scales follows the quarter that used it up.  On the nibble types that form frees
+            // registers nothing uses and is slower (MoE, top-2 of 8 experts, K = 4096: 512 tokens,
+            // N = 14336, Q4_0 236.7 -> 241.9 us, Q4_1 267.0 -> 271.1; 1024 tokens, N = 4096, Q4_1
+            // 171.5 -> 175.7; dense level).
             auto quarter = [&](const i32x16& c, auto iv, int qq, const f32x2& dn) __attribute__((always_inline)) {
                 constexpr int i = decltype(iv)::value;
                 float x[4];
@@ -1044,6 +1052,7 @@ __global__ __launch_bounds__(256, 2) void mmq_planar_kernel(const uint8_t* __res
 #pragma unroll
                 for (int p = 0; p < 4; p++) acc[i][4 * qq + p] = fmaf(edw[qq][p], x[p], acc[i][4 * qq + p]);
             };
+            f32x4 edwn[4];
             f32x2 dnc = *(const f32x2*)&cDn[2 * l32];
 #pragma unroll
             for (int qq = 0; qq < 4; qq++) edw[qq] = *(const f32x4*)&cDw[nbase + 8 * qq];
@@ -1052,7 +1061,7 @@ __global__ __launch_bounds__(256, 2) void mmq_planar_kernel(const uint8_t* __res
             bf = unpack(*(const u32x4*)(cW + woff(0)));
             __builtin_amdgcn_s_setprio(2);
             i32x16 cur = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf, af[0], bias, 0, 0, 0);
-            asm volatile("" : "+v"(cur));
+            if constexpr (BYTES) asm volatile("" : "+v"(cur));
             static_for<NQ>([&](auto qv) __attribute__((always_inline)) {
                 constexpr int q = decltype(qv)::value;
                 constexpr int b = q / TA, i = q % TA;
@@ -1063,7 +1072,12 @@ __global__ __launch_bounds__(256, 2) void mmq_planar_kernel(const uint8_t* __res
                         nxt = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf, af[i + 1], bias, 0, 0, 0);
                     } else {
                         bf = unpack(bxn);
-                        if constexpr (BYTES) asm volatile("" : "+v"(bf), "+v"(af[0]));
+                        if constexpr (BYTES) {
+                            asm volatile("" : "+v"(bf), "+v"(af[0]));
+                        } else {
+#pragma unroll
+                            for (int ii = 0; ii < TA; ii++) af[ii] = afn[ii];
+                        }
                         nxt = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf, af[0], bias, 0, 0, 0);
                     }
                     asm volatile("" : "+v"(nxt));   // pins the issue here, ahead of q's epilogue
@@ -1076,21 +1090,39 @@ __global__ __launch_bounds__(256, 2) void mmq_planar_kernel(const uint8_t* __res
                     constexpr int bn = (q + 1) / TA, in = (q + 1) % TA;
                     dnn = *(const f32x2*)&cDn[2 * (bn * BM + in * 32 + l32)];
                 }
-                if constexpr (b + 1 < KB && i < TA - 1) {
-                    // the fragments whose last MFMA is issued: the next block's into their registers
-                    if constexpr (i == 0) af[0] = *(const i32x4*)(cA + aoff[b + 1]);
-                    af[i + 1] = *(const i32x4*)(cA + (i + 1) * 32 * 128 + aoff[b + 1]);
-                    if constexpr (i == TA - 2) bxn = *(const u32x4*)(cW + woff(b + 1));
-                }
-                if constexpr (i == TA - 1 && b + 1 < KB) edw[0] = *(const f32x4*)&cDw[(b + 1) * BN + nbase];
-                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (BYTES) {
+                    if constexpr (b + 1 < KB && i < TA - 1) {
+                        if constexpr (i == 0) af[0] = *(const i32x4*)(cA + aoff[b + 1]);
+                        af[i + 1] = *(const i32x4*)(cA + (i + 1) * 32 * 128 + aoff[b + 1]);
+                        if constexpr (i == TA - 2) bxn = *(const u32x4*)(cW + woff(b + 1));
+                    }
+                    if constexpr (i == TA - 1 && b + 1 < KB) edw[0] = *(const f32x4*)&cDw[(b + 1) * BN + nbase];
+                    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int qq = 1; qq < 4; qq++) {
-                    quarter(cur, IntC<i>{}, qq, dnc);
-                    if constexpr (i == TA - 1 && b + 1 < KB) edw[qq] = *(const f32x4*)&cDw[(b + 1) * BN + nbase + 8 * qq];
+                    for (int qq = 1; qq < 4; qq++) {
+                        quarter(cur, IntC<i>{}, qq, dnc);
+                        if constexpr (i == TA - 1 && b + 1 < KB) edw[qq] = *(const f32x4*)&cDw[(b + 1) * BN + nbase + 8 * qq];
+                    }
+                    asm volatile("" : "+v"(acc[i]));
+                    __builtin_amdgcn_sched_barrier(0);
+                } else {
+                    if constexpr (i == 0 && b + 1 < KB) {
+#pragma unroll
+                        for (int ii = 0; ii < TA; ii++) afn[ii] = *(const i32x4*)(cA + ii * 32 * 128 + aoff[b + 1]);
+                        bxn = *(const u32x4*)(cW + woff(b + 1));
+                    }
+                    if constexpr (i == TA - 2 && b + 1 < KB) {
+#pragma unroll
+                        for (int qq = 0; qq < 4; qq++) edwn[qq] = *(const f32x4*)&cDw[(b + 1) * BN + nbase + 8 * qq];
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int qq = 1; qq < 4; qq++) quarter(cur, IntC<i>{}, qq, dnc);
+                    if constexpr (i == TA - 1 && b + 1 < KB) {
+#pragma unroll
+                        for (int qq = 0; qq < 4; qq++) edw[qq] = edwn[qq];
+                    }
                 }
-                if constexpr (BYTES) asm volatile("" : "+v"(acc[i]));
-                __builtin_amdgcn_sched_barrier(0);
                 dnc = dnn;
                 cur = nxt;
             });
@@ -1146,8 +1178,11 @@ __global__ __launch_bounds__(256, 2) void mmq_planar_kernel(const uint8_t* __res
         __builtin_amdgcn_s_setprio(0);
         // side term over the step's 4 blocks (f16 MFMA, exact products; k = 4..7 read zeros)
         if constexpr (SIDE) {
-            const u32x2 dwv = *(const u32x2*)&cDh[(wn * 32 + l32) * 4];
-            const f16x4 dw4 = __builtin_bit_cast(f16x4, u32x2{hi ? 0u : dwv.x, hi ? 0u : dwv.y});
+            f16x4 dw4 = *(const f16x4*)&cDh[dh_idx];
+            if constexpr (!ZROW) {
+                const u32x2 v = __builtin_bit_cast(u32x2, dw4);
+                dw4 = __builtin_bit_cast(f16x4, u32x2{hi ? 0u : v.x, hi ? 0u : v.y});
+            }
 #pragma unroll
             for (int i = 0; i < TA; i++) {
                 const f16x4 sa4 = *(const f16x4*)&cSa[(i * 32 + l32) * 4];
@@ -1157,6 +1192,12 @@ __global__ __launch_bounds__(256, 2) void mmq_planar_kernel(const uint8_t* __res
     };
 
     // ---- pipeline ----
+    if constexpr (ZROW) {
+        if (t < 4) {
+            sDh0[BN * 4 + t] = 0;
+            sDh1[BN * 4 + t] = 0;
+        }
+    }
     auto run = [&](auto tav) __attribute__((always_inline)) {
         constexpr int TA = decltype(tav)::value;
         // waves past the computed sub-tiles stage no activation quants (no wave reads them)
