@@ -1580,23 +1580,39 @@ hipError_t launch_mmq(int wtype, int afmt, const uint8_t* W, const uint8_t* A, f
     return launch_splitk_reduce(partials, C, (int64_t)M * N, splits, s);
 }
 
-// The LDS-DMA GEMM takes fp32 activations (block_q8_1, and block_q8s for Q8_0) against the nibble
-// types wherever the 128 x 128 tile is the automatic pick, and against the byte-staged types from a
-// 128 x 128 grid of 300 workgroups on (whole call, us, the register-staged pick vs this kernel: Q8_0
-// M = 2048, N = K = 4096 (512 workgroups) 137 vs 120, M = 512, N = 14336, K = 4096 (448) 121 vs 106,
-// M = 1000, N = 5000, K = 4096 (320) 110 vs 93, M = 2043, N = 9088, K = 1024 98 vs 83; at 256 and 224
-// workgroups level: 75.4 vs 75.9, 110 vs 114; below behind: M = 256, N = 14336 68 vs 77).
+// The LDS-DMA GEMM takes fp32 activations (block_q8_1, and block_q8s for Q8_0): against the nibble
+// types wherever the 128 x 128 tile is the automatic pick, against the byte-staged types where it
+// measured ahead of the register-staged pick.  Whole calls, us, that pick vs this kernel:
+//  * 128 x 128 grids of 384 workgroups on, where the pick has the same tile, but for the shortest
+//    rows, whose quantise launch and few steps decide: Q8_0 M = 2048, N = K = 4096 119 vs 103, M =
+//    512, N = 14336, K = 4096 115 vs 95, M = 1500, N = 4096, K = 1024 36.9 vs 35.1, but K = 256 17.4
+//    vs 17.8, M = 512, N = 14336, K = 256 18.2 vs 20.1, M = 1024, N = 6600, K = 768 28.9 vs 29.7
+//    (past 512 workgroups K = 768 wins: M = 2048, N = 5120 47.6 vs 42.8); Q5_0, whose pick unpacks
+//    more, from K = 512: M = 1024, N = 6600 24.2 vs 23.9, K = 256 18.0 vs 19.3.
+//  * 300 .. 383 workgroups, Q8_0: the pick is the 64 x 64 tile, 768 workgroups at a time and half
+//    the rows of padding, so it loses only where its grid needs well over one such round.  Past 1.5
+//    rounds from K = 4096 on (M = 1000, N = 5000 106 vs 88, M = 330, N = 14336 89.7 vs 87.7; K = 2048
+//    49.4 vs 52.0, M = 1500, N = 3100, K = 1024 30.5 vs 33.6; at 1.4 rounds M = 300, N = 14336, K = 4096
+//    86.0 vs 87.6), past 1.8 from K = 1536 (M = 1280, N = 4800 46.6 vs 44.1; K = 1024 35.4 vs 34.7, M =
+//    1299, N = 4352, K = 1024 32.8 vs 34.9).  One round: M = 40, N = 40000, K = 2048 30.3 vs 49.1.
+//  * Q5_0 and Q5_1 not below 384: that pick adds the s_a term once per 8 blocks, this kernel (as the
+//    128 x 128 pick) per 4, and a result must not depend on whether the caller's workspace holds
+//    the planar form.
+//  * below 300: level or behind (Q8_0 at 256 and 224 workgroups 75.4 vs 75.9, 110 vs 114).
 // Configuration 8 forces it.
 #ifndef KSQ_MMQ_PLANAR
 #define KSQ_MMQ_PLANAR 1
 #endif
-constexpr int kPlanarByteMinWGs = 300;
 bool mmq_planar_preferred(int wtype, int M, int N, int K) {
     if (is_kquant(wtype)) return false;
     if (g_mmq_config == 8) return true;
     if (!KSQ_MMQ_PLANAR || g_mmq_config != 0) return false;
     if (wtype == kWQ40 || wtype == kWQ41) return pick_config(wtype, M, N, K) == 1;
-    return grid_wgs<TileL>(M, N) >= kPlanarByteMinWGs;
+    const int wgs = grid_wgs<TileL>(M, N);
+    if (wgs >= 384) return K >= (wtype != kWQ80 ? 512 : wgs > 512 ? 768 : 1024);
+    if (wtype != kWQ80 || wgs < 300) return false;
+    const int round = kCUCount * TileS::OCC, wgs64 = grid_wgs<TileS>(M, N);
+    return (K >= 4096 && 2 * wgs64 > 3 * round) || (K >= 1536 && 5 * wgs64 > 9 * round);
 }
 
 int mmq_planar_splits(int wtype, int M, int N, int K) { return split_for<TileL>(wtype, M, N, K); }

@@ -247,9 +247,19 @@ def _engine_cases():
                             (129, 129, 256, False)):
             cases.append((f"mmqp_m{M}_k{K}_w{wt}", wt, M, N, K, 0, 2, 8, {"quantize", "mmq_planar"} | ({"splitk"} if sp else set()), 0))
     cases.append(("mmqp_q8s", 1, 140, 200, 768, 2, 2, 8, {"quantize", "mmq_planar"}, 0))
-    # the automatic route at its first grid (300 workgroups of 128 x 128)
+    # the automatic route.  From 384 workgroups of 128 x 128 on, past the shortest rows; 300 of them
+    # with rows of 256 elements are slower there than on the 64 x 64 tile (15.3 vs 17.7 us), as are
+    # grids whose row tiles are mostly padding (M = 40: 313 workgroups, 313 half-tiles of work)
     for wt in (1, 5, 6):
-        cases.append((f"mmqp_auto_w{wt}", wt, 1500, 3100, 256, 0, 0, 0, {"quantize", "mmq_planar"}, 0))
+        cases.append((f"mmqp_auto_w{wt}", wt, 1500, 3100, 256, 0, 0, 0, {"quantize", "mmq3"}, 0))
+        cases.append((f"mmqp_auto_rows40_w{wt}", wt, 40, 40000, 512, 0, 0, 0, {"quantize", "mmq3"}, 0))
+        cases.append((f"mmqp_auto_384_w{wt}", wt, 130, 24500, 1024, 0, 0, 0, {"quantize", "mmq_planar"}, 0))
+        cases.append((f"mmqp_auto_384_short_w{wt}", wt, 130, 24500, 256, 0, 0, 0, {"quantize", "mmq6"}, 0))
+    # Q8_0 (also by block_q8s rules) below 384 where the 64 x 64 grid needs 1.8 rounds of the chip;
+    # the K-step-8 sums of Q5 keep those on the 64 x 64 tile
+    cases.append(("mmqp_auto_375_w1", 1, 65, 48000, 1536, 0, 0, 0, {"quantize", "mmq_planar"}, 0))
+    cases.append(("mmqp_auto_375_q8s", 1, 65, 48000, 1536, 2, 0, 0, {"quantize", "mmq_planar"}, 0))
+    cases.append(("mmqp_auto_375_w5", 5, 65, 48000, 1536, 0, 0, 0, {"quantize", "mmq3"}, 0))
     cases.append(("splitk_w0", 0, 32, 1024, 8192, 1, 2, 0, {"mmq5", "splitk"}, 0))
     cases.append(("splitk_w1", 1, 32, 1024, 8192, 1, 2, 0, {"mmq3", "splitk"}, 0))
     # the native W8A8C8 operator's block_q8s activations: fp32 (its quantiser) and pre-quantised
@@ -504,15 +514,15 @@ def test_dropin_forwarding_module(dev):
     assert D.dropin_forward(b"no_such_entry", None, None, None, 1, 1, 32) == -1
 
 
+@pytest.mark.parametrize("M,N,K", [(1500, 3100, 256), (130, 24500, 1024)])   # the second prefers the planar form
 @pytest.mark.parametrize("wtype", [1, 5, 6])
-def test_byte_types_block_form_workspace(dev, wtype):
+def test_byte_types_block_form_workspace(dev, wtype, M, N, K):
     """A large fp32 call of the byte-staged types with a workspace of the block form's size (36 bytes
     per activation block), smaller than the planar form's, runs in the block form, exactly; with
     one byte less it is refused."""
     import torch
     from ksq import _lib, ops, refcheck
     from oracle import oracle
-    M, N, K = 1500, 3100, 256
     g = np.random.default_rng(4700 + wtype)
     w = refcheck.unit_weights(wtype, g, N, K)
     x = refcheck.unit_activations(g, M, K, qmax=QMAX_F32[wtype], onehot=refcheck.onehot_pattern(M, K // 32))
@@ -528,3 +538,29 @@ def test_byte_types_block_form_workspace(dev, wtype):
     assert np.array_equal(y.cpu().numpy()[:, cols], ref.astype(np.float32))
     with pytest.raises(_lib.KsqError):
         ops.gemm(wtype, 0, _t(w, dev), _t(x, dev), M, N, K, workspace=ws[:need - 1])
+
+
+@pytest.mark.parametrize("wtype,atype,M,N,K", [(wt, at, M, N, K) for wt, at in ((1, 0), (1, 2), (5, 0), (6, 0))
+                                               for M, N, K in ((1500, 3100, 256), (1000, 5000, 4096), (65, 48000, 1536),
+                                                               (130, 24500, 1024), (1500, 4100, 512))])
+def test_byte_types_result_independent_of_workspace(dev, wtype, atype, M, N, K):
+    """The same call with the block form's workspace, with one that holds the planar form, from the
+    library's pool and from the static scratch: the same bits (ordinary values, whose sums
+    round differently in another order)."""
+    import ctypes
+    import torch
+    from ksq import _lib, ops, synth
+    L = _lib.lib()
+    g = np.random.default_rng(4800 + wtype)
+    w, x = _t(synth.weights(wtype, g, N, K), dev), _t(synth.activations(g, M, K), dev)
+    need = ops.workspace_size(wtype, atype, M, N, K)
+    small = torch.empty(need, dtype=torch.uint8, device=dev)
+    large = torch.empty(max(need, L.ksq_debug_planar_bytes(M, K)), dtype=torch.uint8, device=dev)
+    y = [ops.gemm(wtype, atype, w, x, M, N, K, workspace=small), ops.gemm(wtype, atype, w, x, M, N, K, workspace=large),
+         ops.gemm(wtype, atype, w, x, M, N, K)]
+    out = torch.full((M, N), float("nan"), dtype=torch.float32, device=dev)
+    _lib.check(L.ksq_gemm_noalloc(wtype, atype, w.data_ptr(), x.data_ptr(), out.data_ptr(), M, N, K,
+                                  ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    torch.cuda.synchronize()
+    for o in (*y[1:], out):
+        assert torch.equal(o, y[0])
