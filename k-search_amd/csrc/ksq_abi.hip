@@ -55,6 +55,9 @@ int hip_error(hipError_t e, const char* where) {
 // small uses the device's largest pool that is large enough (the usual warm-up-then-capture
 // sequence: the call was made eagerly on another stream first), so such a graph shares that
 // stream's pool and must not run concurrently with its calls.
+// A call that can also do with less scratch names both sizes.  It gets the larger wherever the pool
+// may grow to it; a capturing stream's own pool comes before a borrowed one as soon as it holds the
+// smaller size.
 struct Pool {
     void* ptr = nullptr;
     size_t size = 0;
@@ -63,40 +66,50 @@ struct Pool {
 std::mutex g_pool_mu;
 std::map<std::pair<int, uintptr_t>, Pool> g_pools;
 
-int pool_get(size_t bytes, hipStream_t s, void** out) {
+// *got: the bytes the call may use, at least min_bytes (min_bytes = 0: bytes itself).
+int pool_get(size_t bytes, hipStream_t s, void** out, size_t min_bytes = 0, size_t* got = nullptr) {
+    if (min_bytes == 0 || min_bytes > bytes) min_bytes = bytes;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return hip_error(e, "hipGetDevice");
     std::lock_guard<std::mutex> lk(g_pool_mu);
     Pool& p = g_pools[{dev, (uintptr_t)s}];
+    auto take = [&](const Pool& q) {
+        *out = q.ptr;
+        if (got) *got = q.size;
+        return KSQ_OK;
+    };
     if (p.size < bytes) {
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
         if (s && hipStreamIsCapturing(s, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone) {
+            if (p.size >= min_bytes) return take(p);
             const Pool* big = nullptr;
             for (const auto& kv : g_pools)
-                if (kv.first.first == dev && kv.second.size >= bytes && (!big || kv.second.size > big->size))
+                if (kv.first.first == dev && kv.second.size >= min_bytes && (!big || kv.second.size > big->size))
                     big = &kv.second;
-            if (big) {
-                *out = big->ptr;
-                return KSQ_OK;
-            }
+            if (big) return take(*big);
             return set_error(KSQ_ERR_WORKSPACE,
                              "the workspace pool would have to grow to %zu bytes during graph capture; "
                              "pass a workspace",
-                             bytes);
+                             min_bytes);
         }
         size_t want = 2 * p.size;
         if (want < bytes) want = bytes;
         if (want < (1u << 20)) want = 1u << 20;
         void* np = nullptr;
         e = hipMalloc(&np, want);
+        if (e != hipSuccess && min_bytes < bytes) {   // memory short: the smaller size
+            (void)hipGetLastError();
+            if (p.size >= min_bytes) return take(p);
+            want = min_bytes;
+            e = hipMalloc(&np, want);
+        }
         if (e != hipSuccess) return hip_error(e, "hipMalloc(workspace)");
         if (p.ptr) p.retired.push_back(p.ptr);
         p.ptr = np;
         p.size = want;
     }
-    *out = p.ptr;
-    return KSQ_OK;
+    return take(p);
 }
 
 // ksq_gemm_noalloc's scratch: a file-scope device array (one copy per GPU, allocated with the
@@ -518,25 +531,21 @@ int ksq_gemm(int wtype, int atype, const void* weight, const void* activation, f
     GemmWs L = gemm_ws(wtype, atype, M, N, K, mmq, planar);
     uint8_t* ws = (uint8_t*)workspace;
     if (L.total) {
-        if (ws && planar && workspace_bytes < L.total && planar_optional(wtype)) {
-            planar = false;
-            L = gemm_ws(wtype, atype, M, N, K, mmq, false);
-        }
-        if (ws) {
-            if (workspace_bytes < L.total)
-                return set_error(KSQ_ERR_WORKSPACE, "workspace %zu < %zu bytes", workspace_bytes, L.total);
-            if ((uintptr_t)ws & 15u) return set_error(KSQ_ERR_ALIGN, "workspace must be 16-byte aligned");
-        } else {
+        const bool optional = planar && planar_optional(wtype);
+        const GemmWs B = optional ? gemm_ws(wtype, atype, M, N, K, mmq, false) : L;
+        if (!ws) {
             void* p = nullptr;
-            st = pool_get(L.total, s, &p);
-            if (st == KSQ_ERR_WORKSPACE && planar && planar_optional(wtype)) {
-                planar = false;
-                L = gemm_ws(wtype, atype, M, N, K, mmq, false);
-                st = pool_get(L.total, s, &p);
-            }
+            st = pool_get(L.total, s, &p, B.total, &workspace_bytes);
             if (st != KSQ_OK) return st;
             ws = (uint8_t*)p;
         }
+        if (optional && workspace_bytes < L.total) {
+            planar = false;
+            L = B;
+        }
+        if (workspace_bytes < L.total)
+            return set_error(KSQ_ERR_WORKSPACE, "workspace %zu < %zu bytes", workspace_bytes, L.total);
+        if ((uintptr_t)ws & 15u) return set_error(KSQ_ERR_ALIGN, "workspace must be 16-byte aligned");
     }
     float* partials = L.p ? (float*)(ws + L.q) : nullptr;
     if (planar) {

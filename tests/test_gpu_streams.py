@@ -109,3 +109,43 @@ def test_capture_refuses_to_grow_pool(dev):
     torch.cuda.synchronize()
     assert torch.equal(out, want)
     del graph
+
+
+@pytest.mark.parametrize("larger_pool", [False, True])
+@pytest.mark.parametrize("wtype", [1, 5])
+def test_capture_takes_form_that_own_pool_holds(dev, wtype, larger_pool):
+    """A byte-staged type's prefill call captured without a workspace on a stream whose pool holds the
+    block form and not the larger planar one: the block form in that pool, whether or not another
+    stream's pool would hold the planar form (a borrowed pool would be shared with that stream)."""
+    import torch
+    from ksq import _lib, ops, synth
+    g = np.random.default_rng(6302)
+    M, N, K = 1500, 4100, 1024
+    w = _t(synth.weights(wtype, g, N, K), dev)
+    x = _t(synth.activations(g, M, K), dev)
+    need = ops.workspace_size(wtype, 0, M, N, K)
+    assert need < _lib.lib().ksq_debug_planar_bytes(M, K)
+    out = torch.empty((M, N), dtype=torch.float32, device=dev)
+    want = ops.gemm(wtype, 0, w, x, M, N, K, workspace=torch.empty(need, dtype=torch.uint8, device=dev))
+    torch.cuda.synchronize()
+    _lib.lib().ksq_release()
+    own, other = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(own):
+        ops.gemm(wtype, 4, w, x.half(), M, N, K)    # fp16 rows: the block form's size, no planar form
+    if larger_pool:
+        with torch.cuda.stream(other):
+            ops.gemm(wtype, 0, w, x, M, N, K)
+            assert "mmq_planar" in ops.last_engines()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=own):
+        ops.gemm(wtype, 0, w, x, M, N, K, out=out)
+        eng = ops.last_engines()
+    assert eng == {"quantize", "mmq6"}, eng
+    for _ in range(3):
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+    del graph
