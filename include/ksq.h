@@ -210,7 +210,9 @@ KSQ_API void gemm_w4a32c8_q4_0_fp32_int8_deepseek_v2(const uint8_t* weight, cons
  * accumulation error).  Argument order of the reference launchers: A, B, C.  A 16-byte
  * aligned, finite, |a| < 3.38e38; B and C 4-byte aligned; K % 64 == 0.  workspace: the split-K
  * partial sums, ksq_gemm_w16_workspace_size(M, N, K) bytes (0 when the grid needs no split), or
- * NULL for the library's per-device pool.  Returns a ksq_status. */
+ * NULL for the library's per-device pool.  Above 32 rows a smaller one (a pool under capture, too)
+ * that holds ceil(512 / 128 x 128 tiles) splits of 4 M N bytes is taken as well: the call then
+ * splits less, which is slower and groups the fp32 sums differently.  Returns a ksq_status. */
 KSQ_API size_t ksq_gemm_w16_workspace_size(int M, int N, int K);
 KSQ_API int ksq_gemm_w16(int wtype, const float* A, const uint8_t* B, float* C, int M, int N, int K,
                          void* workspace, size_t workspace_bytes, void* stream);

@@ -424,10 +424,13 @@ int ksq_quantize_q8s(const float* x, uint8_t* y, int M, int K, void* stream) {
     return ok();
 }
 
+static size_t w16_bytes(int splits, int M, int N) {
+    return splits > 1 ? align256((size_t)splits * (size_t)M * (size_t)N * sizeof(float)) : 0;
+}
+
 size_t ksq_gemm_w16_workspace_size(int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
-    const int sp = ksq::w16_splits(M, N, K);
-    return sp > 1 ? align256((size_t)sp * (size_t)M * (size_t)N * sizeof(float)) : 0;
+    return w16_bytes(ksq::w16_splits(M, N, K), M, N);
 }
 
 int ksq_gemm_w16(int wtype, const float* A, const uint8_t* B, float* C, int M, int N, int K, void* workspace,
@@ -450,16 +453,19 @@ int ksq_gemm_w16(int wtype, const float* A, const uint8_t* B, float* C, int M, i
         return set_error(KSQ_ERR_ALIGN, "A must be 16-byte aligned, B and C 4-byte aligned");
     const size_t need = ksq_gemm_w16_workspace_size(M, N, K);
     void* ws = workspace;
+    int max_splits = 1;
     if (need) {
+        const size_t least = w16_bytes(ksq::w16_min_splits(M, N, K), M, N);
         if (ws) {
-            if (workspace_bytes < need) return set_error(KSQ_ERR_WORKSPACE, "workspace %zu < %zu bytes", workspace_bytes, need);
+            if (workspace_bytes < least) return set_error(KSQ_ERR_WORKSPACE, "workspace %zu < %zu bytes", workspace_bytes, least);
             if ((uintptr_t)ws & 15u) return set_error(KSQ_ERR_ALIGN, "workspace must be 16-byte aligned");
         } else {
-            int st = pool_get(need, s, &ws);
+            int st = pool_get(need, s, &ws, least, &workspace_bytes);
             if (st != KSQ_OK) return st;
         }
+        max_splits = (int)((workspace_bytes < need ? workspace_bytes : need) / ((size_t)M * (size_t)N * sizeof(float)));
     }
-    hipError_t e = ksq::launch_w16(wtype, A, B, C, M, N, K, need ? (float*)ws : nullptr, s);
+    hipError_t e = ksq::launch_w16(wtype, A, B, C, M, N, K, need ? (float*)ws : nullptr, max_splits, s);
     return e == hipSuccess ? ok() : hip_error(e, "w16 launch");
 }
 

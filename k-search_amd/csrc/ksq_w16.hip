@@ -654,7 +654,9 @@ struct W16Plan {
 // grid leaves CUs idle, at least 4 steps each.  (Measured, us, best of all tiles and splits / this
 // rule's pick: 64 x 4096 x 4096 19.1 / 19.4; 128 x 14336 x 4096 58 / 58; 512 x 4096 x 4096 59.4 / 59.4;
 // 700 x 3008 x 3008 53.8 / 53.8; 1024 x 4096 x 4096 111 / 111; 218 x 2765 x 18176 92.7 / 95.)
-W16Plan w16_plan(int M, int N, int K) {
+// max_splits: what the caller's scratch holds, the tile then chosen for that.
+W16Plan w16_plan(int M, int N, int K, int max_splits) {
+    if (max_splits > kW16MaxSplits) max_splits = kW16MaxSplits;
     const int steps = K / 64;
     const int grid128 = w16_tiles(M, N, 128, 128);
     if (M <= kW16SmallRows) {
@@ -662,7 +664,7 @@ W16Plan w16_plan(int M, int N, int K) {
         if (wgs >= kW16MinWGs) return {0, 1};
         int sp = (kW16TargetWGs + wgs - 1) / wgs;
         sp = sp < steps / 4 ? sp : steps / 4;
-        sp = sp < kW16MaxSplits ? sp : kW16MaxSplits;
+        sp = sp < max_splits ? sp : max_splits;
         return {0, sp < 1 ? 1 : sp};
     }
     constexpr int cap[4] = {0, 3, 2, 1};
@@ -671,7 +673,7 @@ W16Plan w16_plan(int M, int N, int K) {
     double best_us = 1e30;
     for (int tile = 1; tile <= 3; tile++) {
         const int tiles = w16_tiles(M, N, tile == 1 ? 64 : 128, tile == 3 ? 256 : 128);
-        for (int sp = 1; sp <= kW16MaxSplits; sp++) {
+        for (int sp = 1; sp <= max_splits; sp++) {
             if (sp > 1 && (grid128 >= kW16MinWGs || steps / sp < 4)) break;
             const int per_cu = (int)(((long long)((tiles + 7) / 8) * sp + 31) / 32);   // on the fullest XCD
             const double rounds = (double)(per_cu / cap[tile]) * step_us[tile][cap[tile]] + step_us[tile][per_cu % cap[tile]];
@@ -689,7 +691,17 @@ W16Plan w16_plan(int M, int N, int K) {
 
 int w16_splits(int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0 || w16_uses_gemv(M)) return 1;
-    return w16_plan(M, N, K).splits;
+    return w16_plan(M, N, K, kW16MaxSplits).splits;
+}
+
+// The splits a workspace has to hold: the plan's, or the count that takes the 128 x 128 grid to 512
+// workgroups where that is less.  Workspaces were sized by the latter before the plan had more than
+// one tile; 57 x 10919 x 9472 then took 6 splits where the plan takes 8.
+int w16_min_splits(int M, int N, int K) {
+    const int sp = w16_splits(M, N, K), wgs = M > 0 && N > 0 ? w16_tiles(M, N, 128, 128) : 1;
+    if (sp == 1 || M <= kW16SmallRows) return sp;
+    const int most = (kW16TargetWGs + wgs - 1) / wgs;
+    return sp < most ? sp : most;
 }
 
 template <class T, int WT>
@@ -743,14 +755,14 @@ static hipError_t w16_gemv_dispatch(const float* A, const uint8_t* W, float* C, 
 }
 
 hipError_t launch_w16(int wtype, const float* A, const uint8_t* W, float* C, int M, int N, int K, float* partials,
-                      hipStream_t s) {
+                      int max_splits, hipStream_t s) {
     if (wtype != kWQ40 && wtype != kWQ80) return hipErrorNotSupported;
     if (w16_uses_gemv(M)) {
         note_engine(KSQ_ENG_W16);
         return wtype == kWQ40 ? w16_gemv_dispatch<kWQ40>(A, W, C, M, N, K, s)
                               : w16_gemv_dispatch<kWQ80>(A, W, C, M, N, K, s);
     }
-    const W16Plan plan = w16_plan(M, N, K);
+    const W16Plan plan = w16_plan(M, N, K, max_splits);
     const int splits = plan.splits;
     note_engine(KSQ_ENG_W16 | (splits > 1 ? KSQ_ENG_SPLITK : 0u));
     float* out = C;

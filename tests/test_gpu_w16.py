@@ -167,3 +167,50 @@ def test_w16_three_term_split(dev):
         w[n, b, 2 + e % 16] = 0x89 if e < 16 else 0x98
     y, _ = _run(dev, 0, x, w, M, N, K)
     assert np.array_equal(y, x[:, pick])
+
+
+def _plane_bytes(M, N, splits):
+    return (splits * M * N * 4 + 255) // 256 * 256
+
+
+# (the plan takes 15, 5 and 6 splits)
+@pytest.mark.parametrize("wtype", [0, 1])
+@pytest.mark.parametrize("M,N,K,least", [(34, 6092, 4736, 11), (46, 17713, 1280, 4), (34, 13136, 1920, 5)])
+def test_w16_smaller_workspace_exact(dev, wtype, M, N, K, least):
+    """A workspace, or under capture a pool, that holds fewer splits than the plan takes, but as many as
+    bring the 128 x 128 grid to 512 workgroups: fewer splits, exact results; one byte less is refused."""
+    import torch
+    from ksq import _lib, ops
+    g = np.random.default_rng(950 + wtype)
+    w, vals = _int_weights(wtype, g, N, K)
+    amax = 250 if wtype == 0 else 15
+    x = g.integers(-amax, amax + 1, size=(M, K)).astype(np.float32)
+    want = (x.astype(np.float64) @ vals.astype(np.float64).T).astype(np.float32)
+    assert amax * (8 if wtype == 0 else 128) * K < 2 ** 24
+    assert ops.gemm_w16_workspace_size(M, N, K) > _plane_bytes(M, N, least) and least == -(-512 // -(-N // 128))
+    xt, wt = _t(x, dev), _t(w, dev)
+    ws = torch.empty(_plane_bytes(M, N, least), dtype=torch.uint8, device=dev)
+    assert np.array_equal(ops.gemm_w16(wtype, xt, wt, M, N, K, workspace=ws).cpu().numpy(), want)
+    with pytest.raises(_lib.KsqError) as err:
+        ops.gemm_w16(wtype, xt, wt, M, N, K, workspace=ws[:-1])
+    assert _lib.STATUS[err.value.status] == "KSQ_ERR_WORKSPACE"
+    # a pool of about that size: fewer columns of the same layer
+    n = next(n for n in range(N - 32, 64, -32)
+             if _plane_bytes(M, N, least) <= ops.gemm_w16_workspace_size(M, n, K) < ops.gemm_w16_workspace_size(M, N, K))
+    torch.cuda.synchronize()
+    _lib.lib().ksq_release()
+    own = torch.cuda.Stream()
+    with torch.cuda.stream(own):
+        ops.gemm_w16(wtype, xt, wt[:n], M, n, K)
+    out = torch.empty((M, N), dtype=torch.float32, device=dev)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=own):
+        ops.gemm_w16(wtype, xt, wt, M, N, K, out=out)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy(), want)
+    del graph
