@@ -38,13 +38,16 @@ ENTRY_POINTS = {
 
 
 # torch's current stream as the raw handle: building a torch.cuda.Stream object for it took 2.6 of a
-# small call's 8.3 us of host time (M = 1: 8.9 us a pass, GPU kernel 4.3), this 0.2.
-_raw_stream = torch._C._cuda_getCurrentRawStream
-_device = torch._C._cuda_getDevice
+# small call's 8.3 us of host time (M = 1: 8.9 us a pass, GPU kernel 4.3), this 0.2.  Both names are
+# torch's own and absent from a build without a GPU backend, where the public call raises as before.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_device = getattr(torch._C, "_cuda_getDevice", None)
 
 
 def _stream() -> int:
-    return _raw_stream(_device()) if torch.cuda.is_initialized() else torch.cuda.current_stream().cuda_stream
+    if _raw_stream is None or _device is None or not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_device())
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:

@@ -162,3 +162,20 @@ def test_set_path_validation():
     assert L.ksq_set_path(4) == 4
     assert L.ksq_set_path(3) == 0
     assert L.ksq_set_path(0) == 0
+
+
+def test_ops_import_without_torch_gpu_names(monkeypatch):
+    """ksq.ops imports on a torch build without a GPU backend, whose torch._C has no CUDA names; the
+    stream then comes from torch.cuda.current_stream()."""
+    import importlib.util
+    import types
+    import torch
+    import ksq
+    for name in ("_cuda_getCurrentRawStream", "_cuda_getDevice"):
+        monkeypatch.delattr(torch._C, name, raising=False)
+    path = os.path.join(os.path.dirname(ksq.__file__), "ops.py")
+    spec = importlib.util.spec_from_file_location("ksq.ops_without_gpu_names", path)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=77))
+    assert mod._stream() == 77
