@@ -263,12 +263,12 @@ KSQ_API size_t ksq_debug_stream_read_wg_outputs(size_t bytes, size_t wg_bytes);
 KSQ_API int ksq_debug_stream_read_wg(const void* p, size_t bytes, size_t wg_bytes, uint32_t* out, void* stream);
 
 /* Debug / measurement: the two launches of an fp32 ksq_gemm call that takes the LDS-DMA GEMM
- * (Q4_0 / Q4_1 weights, K % 256 == 0, the 128 x 128-tile shapes), run separately so that the
+ * (weights of a 32-element block type, K % 256 == 0, large grids), run separately so that the
  * GEMM kernel can be timed alone.  ksq_debug_quantize_planar writes the planar block_q8_1
  * activations of x [M][K] (fp32, 16-byte aligned) for weight type wtype into `planar`
  * (ksq_debug_planar_bytes(M, K) bytes, 256-byte aligned): the same blocks as
  * ksq_quantize_q8_1, split into an int8 quant plane [M][K], (d, -12582912 d) fp32 pairs
- * [K/32][Mp] (d = the fp16 scale, divided by 8 for Q4_0) and -s fp16 bits [K/128][Mp][4]
+ * [K/32][Mp] (d = the fp16 scale, divided by 8 for Q4_0, 16 for Q5_0) and -s fp16 bits [K/128][Mp][4]
  * (Mp = M rounded up to 128).  ksq_debug_gemm_planar runs the GEMM on them; it splits along K
  * where ksq_gemm would, with its partial sums in the library's workspace pool.  The two in a
  * row write what ksq_gemm writes for the same fp32 input. */

@@ -607,8 +607,8 @@ size_t ksq_debug_planar_bytes(int M, int K) {
 }
 
 int ksq_debug_quantize_planar(int wtype, const float* x, void* planar, int M, int K, void* stream) {
-    if (wtype != KSQ_W_Q4_0 && wtype != KSQ_W_Q4_1)
-        return set_error(KSQ_ERR_TYPE, "the LDS-DMA GEMM takes Q4_0 and Q4_1 weights (weight type %d)", wtype);
+    if (wtype < KSQ_W_Q4_0 || wtype > KSQ_W_Q5_1 || block_elems(wtype) != 32)
+        return set_error(KSQ_ERR_TYPE, "the LDS-DMA GEMM takes the 32-element block types (weight type %d)", wtype);
     if (M < 0 || K < 0 || K % 256) return set_error(KSQ_ERR_SHAPE, "bad shape M=%d K=%d (K %% 256 == 0)", M, K);
     if (M == 0 || K == 0) return ok();
     if (!x || !planar) return set_error(KSQ_ERR_NULL, "x or planar is NULL");
@@ -622,8 +622,8 @@ int ksq_debug_quantize_planar(int wtype, const float* x, void* planar, int M, in
 int ksq_debug_gemm_planar(int wtype, const void* weight, const void* planar, float* output, int M, int N, int K,
                           void* stream) {
     g_engines = 0;
-    if (wtype != KSQ_W_Q4_0 && wtype != KSQ_W_Q4_1)
-        return set_error(KSQ_ERR_TYPE, "the LDS-DMA GEMM takes Q4_0 and Q4_1 weights (weight type %d)", wtype);
+    if (wtype < KSQ_W_Q4_0 || wtype > KSQ_W_Q5_1 || block_elems(wtype) != 32)
+        return set_error(KSQ_ERR_TYPE, "the LDS-DMA GEMM takes the 32-element block types (weight type %d)", wtype);
     if (M < 0 || N < 0 || K < 0 || K % 256) return set_error(KSQ_ERR_SHAPE, "bad shape M=%d N=%d K=%d", M, N, K);
     if (M == 0 || N == 0 || K == 0) return ok();
     if (!weight || !planar || !output) return set_error(KSQ_ERR_NULL, "weight, planar or output is NULL");

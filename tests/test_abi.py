@@ -179,3 +179,16 @@ def test_ops_import_without_torch_gpu_names(monkeypatch):
     spec.loader.exec_module(mod)
     monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=77))
     assert mod._stream() == 77
+
+
+def test_planar_debug_entries_reject_bad_arguments():
+    """The LDS-DMA GEMM's debug entries take the 32-element block types, rows of K % 256 == 0."""
+    from ksq import _lib
+    L = _lib.lib()
+    for wt in (0, 1, 4, 5, 6):
+        assert L.ksq_debug_quantize_planar(wt, FAKE, FAKE, 4, 128, None) == 2          # K % 256
+        assert L.ksq_debug_quantize_planar(wt, FAKE, FAKE + 16, 4, 256, None) == 3     # planar alignment
+        assert L.ksq_debug_gemm_planar(wt, FAKE, FAKE + 16, FAKE, 4, 4, 256, None) == 3
+    for wt in (-1, 2, 3, 7):
+        assert L.ksq_debug_quantize_planar(wt, FAKE, FAKE, 4, 256, None) == 4
+        assert L.ksq_debug_gemm_planar(wt, FAKE, FAKE, FAKE, 4, 4, 256, None) == 4

@@ -85,10 +85,11 @@ def _planar_planes(buf, M, K):
     return q, dn, sa
 
 
-@pytest.mark.parametrize("wtype,M,K", [(0, 2048, 4096), (4, 300, 1024), (0, 1, 256)])
+@pytest.mark.parametrize("wtype,M,K", [(0, 2048, 4096), (4, 300, 1024), (0, 1, 256), (1, 300, 1024), (5, 129, 256),
+                                         (6, 33, 512)])
 def test_quantize_planar_bit_exact(dev, oracle, wtype, M, K):
     """The LDS-DMA GEMM's planar activations hold exactly the oracle's block_q8_1 blocks: quants,
-    d (divided by 8 for Q4_0) with -12582912 d beside it, and -s; rows past M are zeros."""
+    d (divided by 8 for Q4_0, 16 for Q5_0) with -12582912 d beside it, and -s; rows past M are zeros."""
     import torch
     from ksq import ops
     g = np.random.default_rng(120 + M)
@@ -102,7 +103,7 @@ def test_quantize_planar_bit_exact(dev, oracle, wtype, M, K):
     d16 = blk[:, :, 0:2].copy().view(np.float16)[:, :, 0]
     s16 = blk[:, :, 2:4].copy().view(np.uint16)[:, :, 0]
     assert np.array_equal(q, blk[:, :, 4:].reshape(M, K).view(np.int8))
-    d = d16.astype(np.float32) * np.float32(0.125 if wtype == 0 else 1.0)
+    d = d16.astype(np.float32) * np.float32({0: 1 / 8, 5: 1 / 16}.get(wtype, 1.0))
     assert np.array_equal(dn[:, :M, 0], d.T)
     assert np.array_equal(dn[:, :M, 1], (np.float32(-12582912.0) * d).T)
     want_sa = (s16 ^ 0x8000).T.reshape(K // 128, 4, M).transpose(0, 2, 1)
@@ -110,7 +111,8 @@ def test_quantize_planar_bit_exact(dev, oracle, wtype, M, K):
     assert not dn[:, M:, 0].any() and not dn[:, M:, 1].any()
 
 
-@pytest.mark.parametrize("wtype,M,N,K", [(0, 2048, 4096, 4096), (4, 300, 520, 1280)])
+@pytest.mark.parametrize("wtype,M,N,K", [(0, 2048, 4096, 4096), (4, 300, 520, 1280), (1, 300, 520, 1280),
+                                           (5, 200, 330, 1024), (6, 130, 24500, 1024)])
 def test_planar_halves_equal_fp32_call(dev, wtype, M, N, K):
     """ksq_debug_quantize_planar + ksq_debug_gemm_planar write what the fp32 ksq_gemm call writes,
     bit for bit (the bench times the GEMM half alone)."""
