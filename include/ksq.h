@@ -216,6 +216,9 @@ KSQ_API void gemm_w4a32c8_q4_0_fp32_int8_deepseek_v2(const uint8_t* weight, cons
 KSQ_API size_t ksq_gemm_w16_workspace_size(int M, int N, int K);
 KSQ_API int ksq_gemm_w16(int wtype, const float* A, const uint8_t* B, float* C, int M, int N, int K,
                          void* workspace, size_t workspace_bytes, void* stream);
+/* Debug: the tile and K splits ksq_gemm_w16 takes for a shape: tile (0: 32 x 128, 1: 64 x 128, 2:
+ * 128 x 128, 3: 128 x 256) + 16 * splits, or -1 for the decode form (M <= 4) and empty shapes. */
+KSQ_API int ksq_debug_w16_plan(int M, int N, int K);
 /* The reference launchers' form (stream, pool workspace): gemm_w4a16_naive / gemm_w4a16_tiled
  * (Q4_0) and gemm_w8a16_naive (Q8_0). */
 KSQ_API int ksq_gemm_w4a16(const float* A, const uint8_t* B, float* C, int M, int N, int K, void* stream);

@@ -469,6 +469,8 @@ int ksq_gemm_w16(int wtype, const float* A, const uint8_t* B, float* C, int M, i
     return e == hipSuccess ? ok() : hip_error(e, "w16 launch");
 }
 
+int ksq_debug_w16_plan(int M, int N, int K) { return ksq::w16_plan_code(M, N, K); }
+
 int ksq_gemm_w4a16(const float* A, const uint8_t* B, float* C, int M, int N, int K, void* stream) {
     return ksq_gemm_w16(KSQ_W_Q4_0, A, B, C, M, N, K, nullptr, 0, stream);
 }

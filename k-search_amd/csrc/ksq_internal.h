@@ -187,6 +187,8 @@ hipError_t launch_stream_read(const void* p, size_t bytes, size_t wg_bytes, uint
 // then splits accordingly.
 int w16_splits(int M, int N, int K);
 int w16_min_splits(int M, int N, int K);
+// The tile (0: 32 x 128, 1: 64 x 128, 2: 128 x 128, 3: 128 x 256) + 16 * splits; -1: the decode form.
+int w16_plan_code(int M, int N, int K);
 hipError_t launch_w16(int wtype, const float* A, const uint8_t* W, float* C, int M, int N, int K, float* partials,
                       int max_splits, hipStream_t s);
 

@@ -694,6 +694,12 @@ int w16_splits(int M, int N, int K) {
     return w16_plan(M, N, K, kW16MaxSplits).splits;
 }
 
+int w16_plan_code(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || K <= 0 || w16_uses_gemv(M)) return -1;
+    const W16Plan p = w16_plan(M, N, K, kW16MaxSplits);
+    return p.tile + 16 * p.splits;
+}
+
 // The splits a workspace has to hold: the plan's, or the count that takes the 128 x 128 grid to 512
 // workgroups where that is less.  Workspaces were sized by the latter before the plan had more than
 // one tile; 57 x 10919 x 9472 then took 6 splits where the plan takes 8.

@@ -56,6 +56,7 @@ SIGNATURES = {
     "ksq_quantize_q8f": ([_I, _P, _P, _I, _I, _P], _I),
     "ksq_gemm_w16_workspace_size": ([_I, _I, _I], _SZ),
     "ksq_gemm_w16": ([_I, _P, _P, _P, _I, _I, _I, _P, _SZ, _P], _I),
+    "ksq_debug_w16_plan": ([_I, _I, _I], _I),
     "ksq_gemm_w4a16": ([_P, _P, _P, _I, _I, _I, _P], _I),
     "ksq_gemm_w8a16": ([_P, _P, _P, _I, _I, _I, _P], _I),
     "ksq_quantize_q8_1": ([_P, _P, _I, _I, _P], _I),

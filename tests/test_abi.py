@@ -192,3 +192,14 @@ def test_planar_debug_entries_reject_bad_arguments():
     for wt in (-1, 2, 3, 7):
         assert L.ksq_debug_quantize_planar(wt, FAKE, FAKE, 4, 256, None) == 4
         assert L.ksq_debug_gemm_planar(wt, FAKE, FAKE, FAKE, 4, 4, 256, None) == 4
+
+
+@pytest.mark.parametrize("M,N,K,tile,splits", [(33, 4096, 4096, 1, 16), (1024, 4096, 4096, 2, 1), (512, 4096, 4096, 3, 4),
+                                               (700, 3008, 3008, 3, 3), (2048, 4096, 4096, 3, 1), (32, 4096, 4096, 0, 16)])
+def test_w16_plan(M, N, K, tile, splits):
+    """The tile and K splits of the dequantise-then-fp32 GEMM, and the workspace that goes with them."""
+    from ksq import _lib
+    L = _lib.lib()
+    assert L.ksq_debug_w16_plan(M, N, K) == tile + 16 * splits
+    assert L.ksq_gemm_w16_workspace_size(M, N, K) == (splits * M * N * 4 + 255) // 256 * 256 * (splits > 1)
+    assert L.ksq_debug_w16_plan(4, N, K) == -1 and L.ksq_debug_w16_plan(0, N, K) == -1

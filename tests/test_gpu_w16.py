@@ -135,8 +135,8 @@ def test_w16_baseline_shapes(dev, oracle):
             assert _rel_err(y.cpu().numpy()[rows], ref) < TOL, (entry, M)
 
 
-# the 64 x 128, 128 x 128 and 128 x 256 tiles at their edges: one row past the small-batch form, rows and
-# columns one short of and one past a tile, one K step, an odd number of K steps, split along K
+# one row past the small-batch form, rows and columns one short of and one past a tile, one K step, an odd
+# number of K steps, split along K: the 64 x 128 tile's edges but for (2047, 4095, 64), which takes 128 x 256
 @pytest.mark.parametrize("wtype", [0, 1])
 @pytest.mark.parametrize("M,N,K", [(33, 1, 64), (64, 127, 128), (65, 129, 64), (33, 200, 1088), (257, 383, 192),
                                    (1000, 4100, 128), (1025, 4097, 64), (2047, 4095, 64), (2048, 4097, 192)])
@@ -152,21 +152,51 @@ def test_w16_tile_edges_exact(dev, wtype, M, N, K):
     assert "w16" in eng
 
 
-def test_w16_three_term_split(dev):
+# M, N, K, tile (1: 64 x 128, 2: 128 x 128, 3: 128 x 256), splits: each tile's edges in rows and columns, one
+# K step, an odd and an even number of them, split along K into equal and unequal parts
+TILE_CASES = [(65, 129, 704, 1, 2), (63, 161, 512, 1, 2),
+              (383, 5503, 64, 2, 1), (257, 6529, 128, 2, 1), (3327, 513, 192, 2, 1), (2687, 129, 1024, 2, 4),
+              (127, 5247, 1536, 2, 5),
+              (385, 14113, 64, 3, 1), (385, 14081, 128, 3, 1), (3327, 1793, 192, 3, 1), (639, 3327, 1152, 3, 3),
+              (257, 6655, 1024, 3, 3)]
+
+
+@pytest.mark.parametrize("wtype", [0, 1])
+@pytest.mark.parametrize("M,N,K,tile,splits", TILE_CASES)
+def test_w16_every_tile_exact(dev, wtype, M, N, K, tile, splits):
+    """The tile and split count that the shape is listed for, and exact integer results."""
+    from ksq import _lib
+    assert _lib.lib().ksq_debug_w16_plan(M, N, K) == tile + 16 * splits
+    g = np.random.default_rng(930 + M + wtype)
+    w, vals = _int_weights(wtype, g, N, K)
+    amax = 250 if wtype == 0 else 15
+    x = g.integers(-amax, amax + 1, size=(M, K)).astype(np.float32)
+    assert amax * (8 if wtype == 0 else 128) * K < 2 ** 24
+    # exact in fp32 in any order: every partial sum is an integer below 2^24
+    want = x @ vals.astype(np.float32).T
+    y, eng = _run(dev, wtype, x, w, M, N, K, workspace=True)
+    assert np.array_equal(y, want), float(np.abs(y - want).max())
+    assert eng == {"w16"} | ({"splitk"} if splits > 1 else set()), eng
+
+
+@pytest.mark.parametrize("M,N,K,tile", [(130, 300, 256, 1), (257, 6529, 128, 2), (385, 14081, 128, 3)])
+def test_w16_three_term_split(dev, M, N, K, tile):
     """Activations that need all 24 bits: a = 2^23 + odd integers against quants of -1, 0 and 1 (Q4_0
-    nibbles 7, 8, 9), one non-zero per row, so every output is one activation, exactly."""
-    M, N, K = 130, 300, 256
+    nibbles 7, 8, 9), one non-zero per row, so every output is plus or minus one activation, exactly."""
+    from ksq import _lib
+    assert _lib.lib().ksq_debug_w16_plan(M, N, K) % 16 == tile
     g = np.random.default_rng(77)
     x = (g.integers(2 ** 23, 2 ** 24, size=(M, K)) | 1).astype(np.float32) * g.choice([-1.0, 1.0], size=(M, K)).astype(np.float32)
     w = np.zeros((N, K // 32, 18), np.uint8)
     w[..., 0:2] = np.frombuffer(np.float16(1).tobytes(), np.uint8)
     w[..., 2:] = 0x88
-    pick = g.integers(0, K, size=N)
+    pick, sign = g.integers(0, K, size=N), g.choice([-1, 1], size=N)
     for n, k in enumerate(pick):
         b, e = divmod(int(k), 32)
-        w[n, b, 2 + e % 16] = 0x89 if e < 16 else 0x98
+        q = 8 + int(sign[n])
+        w[n, b, 2 + e % 16] = 0x80 | q if e < 16 else q << 4 | 8
     y, _ = _run(dev, 0, x, w, M, N, K)
-    assert np.array_equal(y, x[:, pick])
+    assert np.array_equal(y, x[:, pick] * sign.astype(np.float32))
 
 
 def _plane_bytes(M, N, splits):
