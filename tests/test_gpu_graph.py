@@ -59,6 +59,10 @@ def _replays_match(fn, out, engines_must=None):
 GEMM_CASES = [
     ("planar_q4_0", 0, 0, 2048, 2048, 4096, 0, {"quantize", "mmq_planar"}),     # LDS-DMA GEMM
     ("planar_splitk_q4_1", 4, 0, 300, 520, 1280, 8, {"quantize", "mmq_planar", "splitk"}),
+    # the byte-staged types' planar form, in the larger workspace that it needs
+    ("planar_q8_0", 1, 0, 1500, 4100, 1024, 0, {"quantize", "mmq_planar"}),
+    ("planar_q8_0_q8s", 1, 2, 1500, 4100, 1024, 0, {"quantize", "mmq_planar"}),
+    ("planar_q5_1", 6, 0, 1500, 4100, 1024, 0, {"quantize", "mmq_planar"}),
     ("tile128_q8_1_input", 0, 1, 512, 2048, 4096, 1, {"mmq1"}),
     ("decode_fused_fp32", 0, 0, 1, 4096, 4096, 0, {"gemv_direct_fq"}),
     ("q8_0_m32_splitk", 1, 0, 32, 4096, 8192, 0, {"quantize", "splitk"}),
@@ -79,7 +83,10 @@ def test_gemm_graph_replays(dev, name, wtype, atype, M, N, K, cfg, engines):
     L = _lib.lib()
     assert L.ksq_set_mmq_config(cfg) == 0
     try:
-        ws = torch.empty(max(256, ops.workspace_size(wtype, atype, M, N, K)), dtype=torch.uint8, device=dev)
+        nbytes = max(256, ops.workspace_size(wtype, atype, M, N, K))
+        if "mmq_planar" in engines:
+            nbytes = max(nbytes, L.ksq_debug_planar_bytes(M, K))
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
         out = torch.empty((M, N), dtype=torch.float32, device=dev)
         _replays_match(lambda: ops.gemm(wtype, atype, w, x, M, N, K, out=out, workspace=ws), out, engines)
     finally:

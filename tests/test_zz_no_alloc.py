@@ -89,3 +89,23 @@ def test_noalloc_rejects_calls_past_its_scratch(dev):
     assert _noalloc(0, 1, w, a, y, M, N, K) == 0
     torch.cuda.synchronize()
     assert bool((y == 0.0).all())
+
+
+@pytest.mark.parametrize("wtype", [1, 5, 6])
+def test_noalloc_byte_types_block_form(dev, wtype):
+    """A byte-staged type's prefill call whose planar form is larger than the scratch and whose block form
+    is not runs in the block form, with ksq_gemm's result (which has the planar form's pool)."""
+    import torch
+    from ksq import _lib, ops, synth
+    L = _lib.lib()
+    M, N, K = 6528, 1020, 4096          # 30.1 MB of block_q8_1 blocks, 35.1 MB as planes
+    assert L.ksq_gemm_workspace_size(wtype, 0, M, N, K) <= _lib.NOALLOC_SCRATCH_BYTES < L.ksq_debug_planar_bytes(M, K)
+    g = np.random.default_rng(5200 + wtype)
+    w, x = _t(synth.weights(wtype, g, N, K), dev), _t(synth.activations(g, M, K), dev)
+    y = torch.full((M, N), float("nan"), dtype=torch.float32, device=dev)
+    assert _noalloc(wtype, 0, w, x, y, M, N, K) == 0
+    assert ops.last_engines() == {"quantize", "mmq6"}
+    want = ops.gemm(wtype, 0, w, x, M, N, K)
+    assert ops.last_engines() == {"quantize", "mmq_planar"}
+    torch.cuda.synchronize()
+    assert torch.equal(y, want)
