@@ -997,9 +997,8 @@ __global__ __launch_bounds__(256, 2) void mmq_planar_kernel(const uint8_t* __res
     for (int b = 0; b < KB; b++) aoff[b] = l32 * 128 + (((2 * b + hi) ^ ((l32 >> 1) & 7)) << 4);
     // this lane's weight piece of block b: 16 packed bytes (nibbles, unpacked per fragment) or the
     // 16 int8 of its half
-    auto woff = [&](int b) __attribute__((always_inline)) -> int {
-        return BYTES ? wn * 32 * 128 + aoff[b] : (wn * 32 + l32) * WP + b * 16;
-    };
+    const int wrow = BYTES ? wn * 32 * 128 : (wn * 32 + l32) * WP;
+    auto woff = [&](int b) __attribute__((always_inline)) -> int { return BYTES ? wrow + aoff[b] : wrow + b * 16; };
     const int dh_idx = (ZROW && hi) ? BN * 4 : (wn * 32 + l32) * 4;
     const int nbase = wn * 32 + 4 * hi;   // local weight row of r = 0
 
