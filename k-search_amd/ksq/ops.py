@@ -43,11 +43,12 @@ ENTRY_POINTS = {
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 _device = getattr(torch._C, "_cuda_getDevice", None)
 
-
-def _stream() -> int:
-    if _raw_stream is None or _device is None or not torch.cuda.is_initialized():
+if _raw_stream is not None and _device is not None:
+    def _stream() -> int:
+        return _raw_stream(_device()) if torch.cuda.is_initialized() else torch.cuda.current_stream().cuda_stream
+else:
+    def _stream() -> int:
         return torch.cuda.current_stream().cuda_stream
-    return _raw_stream(_device())
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
