@@ -15,7 +15,8 @@
 //    |a| below the largest bf16).  The weight quants (q - 8 for Q4_0, q for Q8_0) are integers
 //    of at most 8 bits, exact in bf16.  So every product of v_mfma_f32_32x32x16_bf16 is exact
 //    and only the fp32 sums round, as in the reference's fp32 loop (in another order).  The
-//    terms go in smallest first: lo, mid, hi.
+//    terms go in smallest first: lo, mid, hi.  (Above 32 rows Q4_0 is staged as (q - 8) / 16, which
+//    v_cvt_off_f32_i4 gives in one operation, with the scale 16 d: powers of two, exact.)
 //  * Per 32-element block, six MFMAs (three terms x two 16-element halves) give the block's partial
 //    sum P = sum_k a_k q_k for a 32 x 32 patch, then acc = fma(d_w, P, acc): one VALU op per output
 //    and block (the reference multiplies d_w into every weight element instead; the same value up
@@ -28,10 +29,11 @@
 //    sums are added in split order by the int8 GEMM's split-K reduction (deterministic).
 //  * Bound: the chip's power.  Six MFMAs take 198 cycles per patch and block, and at full rate with
 //    random operands the clock falls from 2.4 to about 2 GHz; every instruction beside them costs
-//    time.  M = 2048, N = K = 4096, Q4_0: 183 us (343 TFLOP/s of fp32-exact products, 1.03 PFLOP/s
+//    time.  M = 2048, N = K = 4096, Q4_0: 183 us (375 TFLOP/s of fp32-exact products, 1.13 PFLOP/s
 //    on the bf16 pipe), of it 138 the MFMAs with their LDS reads alone, 12 the epilogue and about
 //    35 the conversions (230 us on single-buffered 128 x 128 tiles with 144-byte row pitch and two
-//    barriers per two blocks).  M = 395, N = 3871, K = 1344: 25.4 us (65.5).
+//    barriers per two blocks); Q8_0, whose weights are twice the bytes to convert, 195 (224).  M =
+//    395, N = 3871, K = 1344: Q4_0 25.4 us (65.5), Q8_0 23.7 (64.2).
 //  * Measured, level or slower: three buffers with the next block's first fragments read ahead of
 //    the barrier, and activation loads four blocks ahead (187-195 us).
 //  * Rows / columns past M or N load a clamped in-range row and are not stored.
@@ -49,7 +51,8 @@ struct W16Tile {
     static constexpr int WN = BN / (32 * TN);   // waves along N
     static constexpr int WM = BM / (32 * TM);   // waves along M
     static constexpr int NT = 64 * WN * WM;     // threads per workgroup
-    static constexpr int AC = (BM * 4 + NT - 1) / NT;   // 8-float activation chunks per thread and block
+    static constexpr int AC = BM * 4 / NT;      // 8-float activation chunks per thread and block
+    static_assert(BM * 4 % NT == 0, "every thread stages whole activation chunks");
     static_assert(NT == 2 * BN, "a thread stages half a weight block per row");
 };
 using W16Huge = W16Tile<128, 256, 2, 2>;
@@ -126,24 +129,21 @@ __global__ __launch_bounds__(T::NT, 2) void w16_kernel(const uint8_t* __restrict
 #pragma unroll
     for (int i = 0; i < AC; i++) {
         const int c = t + NT * i, r = c >> 2, q = c & 3;
-        asrc[i] = A + (size_t)min(m0 + min(r, BM - 1), M - 1) * K + 8 * q;
+        asrc[i] = A + (size_t)min(m0 + r, M - 1) * K + 8 * q;
         // rows of a fragment are XORed with twice the chunk number: the 8 lanes of a write (2 rows
         // x 4 chunks, whose fragments lie multiples of 512 bytes apart) then hit 8 bank groups
         adst[i] = (uint32_t)((r >> 5) * 6144 + (q >> 1) * 1024 + (q & 1) * 512 + (((r & 31) ^ (2 * q)) << 4));
     }
-    const bool a_on = BM * 4 >= NT || t < BM * 4;
     const int wr = t % BN, wh = t / BN;
     const uint8_t* wrow = W + (size_t)min(n0 + wr, N - 1) * nb * BB;
     f32x4 pa[2][AC][2];        // blocks k + 1 and k + 2 while block k is multiplied
     uint32_t pw[WW];           // the weights of two blocks
     auto load_a = [&](auto bv, int kb) __attribute__((always_inline)) {
         constexpr int b = decltype(bv)::value;
-        if (a_on) {
 #pragma unroll
-            for (int i = 0; i < AC; i++) {
-                pa[b][i][0] = *(const f32x4*)(asrc[i] + (size_t)kb * 32);
-                pa[b][i][1] = *(const f32x4*)(asrc[i] + (size_t)kb * 32 + 4);
-            }
+        for (int i = 0; i < AC; i++) {
+            pa[b][i][0] = *(const f32x4*)(asrc[i] + (size_t)kb * 32);
+            pa[b][i][1] = *(const f32x4*)(asrc[i] + (size_t)kb * 32 + 4);
         }
     };
     // the weight bytes of step s (two blocks) that this thread converts.  Q4_0 (36 bytes: d at 0
@@ -166,21 +166,19 @@ __global__ __launch_bounds__(T::NT, 2) void w16_kernel(const uint8_t* __restrict
     // chunk i of the activation block in pa[b], as three bf16 terms, into buffer b
     auto store_a = [&](auto bv, int i, uint8_t* buf) __attribute__((always_inline)) {
         constexpr int b = decltype(bv)::value;
-        if (a_on) {
-            uint32_t ph[4], pm[4], pl[4];
+        uint32_t ph[4], pm[4], pl[4];
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const float a0 = pa[b][i][j >> 1][2 * (j & 1)], a1 = pa[b][i][j >> 1][2 * (j & 1) + 1];
-                ph[j] = bf16_pair(a0, a1);
-                const float r0 = a0 - bf16_low_f32(ph[j]), r1 = a1 - bf16_high_f32(ph[j]);
-                pm[j] = bf16_pair(r0, r1);
-                pl[j] = bf16_pair(r0 - bf16_low_f32(pm[j]), r1 - bf16_high_f32(pm[j]));
-            }
-            uint8_t* d = buf + adst[i];
-            *(u32x4*)d = u32x4{pl[0], pl[1], pl[2], pl[3]};
-            *(u32x4*)(d + 2048) = u32x4{pm[0], pm[1], pm[2], pm[3]};
-            *(u32x4*)(d + 4096) = u32x4{ph[0], ph[1], ph[2], ph[3]};
+        for (int j = 0; j < 4; j++) {
+            const float a0 = pa[b][i][j >> 1][2 * (j & 1)], a1 = pa[b][i][j >> 1][2 * (j & 1) + 1];
+            ph[j] = bf16_pair(a0, a1);
+            const float r0 = a0 - bf16_low_f32(ph[j]), r1 = a1 - bf16_high_f32(ph[j]);
+            pm[j] = bf16_pair(r0, r1);
+            pl[j] = bf16_pair(r0 - bf16_low_f32(pm[j]), r1 - bf16_high_f32(pm[j]));
         }
+        uint8_t* d = buf + adst[i];
+        *(u32x4*)d = u32x4{pl[0], pl[1], pl[2], pl[3]};
+        *(u32x4*)(d + 2048) = u32x4{pm[0], pm[1], pm[2], pm[3]};
+        *(u32x4*)(d + 4096) = u32x4{ph[0], ph[1], ph[2], ph[3]};
     };
     // block b of the step in pw into weight buffer b
     auto store_w = [&](auto bv, uint8_t* buf) __attribute__((always_inline)) {
@@ -649,11 +647,16 @@ struct W16Plan {
 
 // Up to 32 rows: the 32 x 128 tile, split along K to 512 workgroups.  Above: the tile and split
 // with the least predicted time.  A workgroup's step of two blocks takes, with 1, 2, 3 workgroups
-// on a CU (measured, us): 64 x 128 1.07, 1.86, 2.6; 128 x 128 1.7, 3.05; 128 x 256 2.85; a split
+// on a CU (us; measured with K = 8192 and one full round, Q4_0 / Q8_0): 64 x 128 1.07, 1.75, 2.44 /
+// 1.01, 1.89, 2.77; 128 x 128 1.62, 2.88 / 1.70, 3.10; 128 x 256 2.65 / 2.90.  The constants lie between
+// the two types: only the tiles' proportions matter to the pick, and those they share.  A split
 // adds the reduction launch (2.5 us) and its traffic at 4 TB/s.  Splits only where the 128 x 128
-// grid leaves CUs idle, at least 4 steps each.  (Measured, us, best of all tiles and splits / this
-// rule's pick: 64 x 4096 x 4096 19.1 / 19.4; 128 x 14336 x 4096 58 / 58; 512 x 4096 x 4096 59.4 / 59.4;
-// 700 x 3008 x 3008 53.8 / 53.8; 1024 x 4096 x 4096 111 / 111; 218 x 2765 x 18176 92.7 / 95.)
+// grid leaves CUs idle, at least 4 steps each.  Measured, us, best of all tiles and splits / this
+// rule's pick, Q4_0 and Q8_0: 64 x 4096 x 4096 18.0 / 17.9 and 17.7 / 17.8; 128 x 14336 x 4096 52.6 /
+// 53.8 and 56.7 / 57.7; 512 x 4096 x 4096 56.7 / 57.6 and 60.9 / 61.5; 700 x 3008 x 3008 52.4 / 53.3 and
+// 56.4 / 56.6; 1024 x 4096 x 4096 level; 218 x 2765 x 18176 level; 2048 x 4096 x 4096 level.  Over 36
+// shapes the pick is within 4% of the best for 33 (Q4_0) and 30 (Q8_0); the worst, both types: 88 x
+// 1947 x 4992 17.9 / 20.0, 256 x 4096 x 4096 36.4 / 39.7.
 // max_splits: what the caller's scratch holds, the tile then chosen for that.
 W16Plan w16_plan(int M, int N, int K, int max_splits) {
     if (max_splits > kW16MaxSplits) max_splits = kW16MaxSplits;
