@@ -56,7 +56,7 @@ TRAFFIC = {
     "moe_q4_0_T512_E8_top2": (int(((199520.0 + 4149.3 + 35.1) * 2.0 + 57344.0 + 5641.1 + 28688.2) * 1024),
                               "profiles/moe_q4_0_t512_e8_top2.md"),
     "w4a16_q4_0_M1": (int((4732.8 * 2.0 + 16.0) * 1024), "profiles/w16_q4_0_m1_m2048_n4096_k4096.md"),
-    "w4a16_q4_0_M2048": (int((53707.2 * 2.0 + 32768.0) * 1024), "profiles/w16_q4_0_m1_m2048_n4096_k4096.md"),
+    "w4a16_q4_0_M2048": (int((53322.4 * 2.0 + 32768.0) * 1024), "profiles/w16_q4_0_m1_m2048_n4096_k4096.md"),
     "deepseek_v2_q8f_q4_0_M2048": (int(((45713.1 + 16437.1) * 2.0 + 32768.0 + 10240.0) * 1024),
                                    "profiles/q8f_q4_0_m2048_n4096_k4096.md"),
     "deepseek_v2_q8f_q4_0_M1": (int((4727.9 * 2.0 + 16.0) * 1024), "profiles/q8f_q4_0_m2048_n4096_k4096.md"),
