@@ -225,10 +225,15 @@ KSQ_API int ksq_gemm_w4a16(const float* A, const uint8_t* B, float* C, int M, in
 KSQ_API int ksq_gemm_w8a16(const float* A, const uint8_t* B, float* C, int M, int N, int K, void* stream);
 
 /* Workspace bytes ksq_gemm needs for (wtype, atype, M, N, K): the quantised copy of fp32 or
- * fp16 activations (block_q8_1 rows, or the LDS-DMA GEMM's planar form for fp32 activations
- * at large M, 42 bytes per block; for Q8_0, Q5_0 and Q5_1 the block form's 36 bytes, and a call
- * whose workspace holds 42 takes the faster planar form), plus the split-K partial sums of small MFMA grids (so it can
- * be non-zero for pre-quantised activations too).  The workspace must be 16-byte aligned. */
+ * fp16 activations (block_q8_1 rows, 36 bytes per block, or for fp32 activations against Q4_0 / Q4_1
+ * at large M the LDS-DMA GEMM's planar form, 42), plus the split-K partial sums of small MFMA
+ * grids (so it can be non-zero for pre-quantised activations too).  The workspace must be 16-byte
+ * aligned.
+ * For Q8_0, Q5_0 and Q5_1 weights the size is the block form's throughout.  Where the LDS-DMA GEMM
+ * serves them (large grids, fp32 input) a call takes its faster planar form if the workspace, the
+ * library pool or the static scratch holds that: ksq_debug_planar_bytes(M, K) bytes.  So pass the
+ * larger of the two sizes (Q8_0, M = 512, N = 14336, K = 4096: 93 us, with the block form's size
+ * 115).  The results are the same bits in either form. */
 KSQ_API size_t ksq_gemm_workspace_size(int wtype, int atype, int M, int N, int K);
 
 /* General entry: wtype = enum ksq_wtype, atype = enum ksq_atype (the block_q8s forms pair

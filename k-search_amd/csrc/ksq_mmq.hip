@@ -825,8 +825,8 @@ __device__ __forceinline__ void wait_vmem_all() { asm volatile("s_waitcnt vmcnt(
 // rows, swizzled pieces), so a fragment needs no unpacking.  Without the unpack between the reads
 // and the MFMAs the compiler ran a step's MFMAs ahead of their epilogues and its FMAs behind them
 // (600 registers spilled); empty asm statements on the fragments and on each sub-tile's accumulators
-// hold them to their region: no spill, Q8_0 M = 2048, N = K = 4096 95 us, M = 512, N = 14336, K = 4096 97
-// (GEMM alone; register-staged 128 x 128 tile 110).
+// hold them to their region: no spill.  GEMM alone, us, against the register-staged 128 x 128 tile: Q8_0 M =
+// 2048, N = K = 4096 95 vs 112, M = 512, N = 14336, K = 4096 90 vs 109; Q5_0 96 vs 111 and 91 vs 110; Q5_1 as Q5_0.
 // Bound (Q4_0 M = 2048, N = K = 4096, timing-only variants on one box, GEMM 88.5 us): the vector pipe and
 // the MFMAs alone 69, their LDS reads 5, the global loads 10; without the MFMAs 78.
 // MOE (the expert-grouped GEMM): workgroup y is entry y of the tile schedule (128-row tiles of one

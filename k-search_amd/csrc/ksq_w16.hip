@@ -32,7 +32,7 @@
 //    time.  M = 2048, N = K = 4096, Q4_0: 183 us (375 TFLOP/s of fp32-exact products, 1.13 PFLOP/s
 //    on the bf16 pipe), of it 138 the MFMAs with their LDS reads alone, 12 the epilogue and about
 //    35 the conversions (230 us on single-buffered 128 x 128 tiles with 144-byte row pitch and two
-//    barriers per two blocks); Q8_0, whose weights are twice the bytes to convert, 195 (224).  M =
+//    barriers per two blocks); Q8_0, whose weights are twice the bytes to convert, 197 (224).  M =
 //    395, N = 3871, K = 1344: Q4_0 25.4 us (65.5), Q8_0 23.7 (64.2).
 //  * Measured, level or slower: three buffers with the next block's first fragments read ahead of
 //    the barrier, and activation loads four blocks ahead (187-195 us).
