@@ -1588,6 +1588,12 @@ hipError_t launch_mmq(int wtype, int afmt, const uint8_t* W, const uint8_t* A, f
 //    vs 17.8, M = 512, N = 14336, K = 256 18.2 vs 20.1, M = 1024, N = 6600, K = 768 28.9 vs 29.7
 //    (past 512 workgroups K = 768 wins: M = 2048, N = 5120 47.6 vs 42.8); Q5_0, whose pick unpacks
 //    more, from K = 512: M = 1024, N = 6600 24.2 vs 23.9, K = 256 18.0 vs 19.3.
+//    This kernel computes all 128 rows of the last row tile, the pick's upper waves skip theirs: with at
+//    most 64 rows there it is ahead from K = 3072 on with two row tiles (Q8_0 M = 132, N = 32768, K = 1536
+//    53.5 vs 64.4, K = 2048 69.1 vs 74.5, K = 3072 level, K = 4096 ahead by 2-20%), from 2048 with three
+//    to seven (M = 260, N = 21760, K = 768 50.9 vs 63.3, K = 1024 63.2 vs 69.9, K = 1536 level, K = 2048
+//    ahead by 4-15%) and from 1024 past that; one row tile is never behind.  Over 3400 shapes of
+//    388 .. 1008 workgroups, K = 512 .. 7168, Q8_0 and Q5_0.
 //  * 300 .. 383 workgroups, Q8_0: the pick is the 64 x 64 tile, 768 workgroups at a time and half
 //    the rows of padding, so it loses only where its grid needs well over one such round.  Past 1.5
 //    rounds from K = 4096 on (M = 1000, N = 5000 106 vs 88, M = 330, N = 14336 89.7 vs 87.7; K = 2048
@@ -1608,7 +1614,11 @@ bool mmq_planar_preferred(int wtype, int M, int N, int K) {
     if (!KSQ_MMQ_PLANAR || g_mmq_config != 0) return false;
     if (wtype == kWQ40 || wtype == kWQ41) return pick_config(wtype, M, N, K) == 1;
     const int wgs = grid_wgs<TileL>(M, N);
-    if (wgs >= 384) return K >= (wtype != kWQ80 ? 512 : wgs > 512 ? 768 : 1024);
+    if (wgs >= 384) {
+        const int mt = (M + TileL::BM - 1) / TileL::BM, last = M - (mt - 1) * TileL::BM;
+        if (mt > 1 && last <= 64 && K < (mt == 2 ? 3072 : mt < 8 ? 2048 : 1024)) return false;
+        return K >= (wtype != kWQ80 ? 512 : wgs > 512 ? 768 : 1024);
+    }
     if (wtype != kWQ80 || wgs < 300) return false;
     const int round = kCUCount * TileS::OCC, wgs64 = grid_wgs<TileS>(M, N);
     return (K >= 4096 && 2 * wgs64 > 3 * round) || (K >= 1536 && 5 * wgs64 > 9 * round);

@@ -253,8 +253,9 @@ def _engine_cases():
     for wt in (1, 5, 6):
         cases.append((f"mmqp_auto_w{wt}", wt, 1500, 3100, 256, 0, 0, 0, {"quantize", "mmq3"}, 0))
         cases.append((f"mmqp_auto_rows40_w{wt}", wt, 40, 40000, 512, 0, 0, 0, {"quantize", "mmq3"}, 0))
-        cases.append((f"mmqp_auto_384_w{wt}", wt, 130, 24500, 1024, 0, 0, 0, {"quantize", "mmq_planar"}, 0))
+        cases.append((f"mmqp_auto_384_w{wt}", wt, 193, 24500, 1024, 0, 0, 0, {"quantize", "mmq_planar"}, 0))
         cases.append((f"mmqp_auto_384_short_w{wt}", wt, 130, 24500, 256, 0, 0, 0, {"quantize", "mmq6"}, 0))
+        cases.append((f"mmqp_auto_384_last2_w{wt}", wt, 130, 24500, 1024, 0, 0, 0, {"quantize", "mmq6"}, 0))
     # Q8_0 (also by block_q8s rules) below 384 where the 64 x 64 grid needs 1.8 rounds of the chip;
     # the K-step-8 sums of Q5 keep those on the 64 x 64 tile
     cases.append(("mmqp_auto_375_w1", 1, 65, 48000, 1536, 0, 0, 0, {"quantize", "mmq_planar"}, 0))
@@ -514,7 +515,7 @@ def test_dropin_forwarding_module(dev):
     assert D.dropin_forward(b"no_such_entry", None, None, None, 1, 1, 32) == -1
 
 
-@pytest.mark.parametrize("M,N,K", [(1500, 3100, 256), (130, 24500, 1024)])   # the second prefers the planar form
+@pytest.mark.parametrize("M,N,K", [(1500, 3100, 256), (193, 24500, 1024)])   # the second prefers the planar form
 @pytest.mark.parametrize("wtype", [1, 5, 6])
 def test_byte_types_block_form_workspace(dev, wtype, M, N, K):
     """A large fp32 call of the byte-staged types with a workspace of the block form's size (36 bytes
@@ -540,9 +541,26 @@ def test_byte_types_block_form_workspace(dev, wtype, M, N, K):
         ops.gemm(wtype, 0, _t(w, dev), _t(x, dev), M, N, K, workspace=ws[:need - 1])
 
 
+@pytest.mark.parametrize("wtype,atype", [(1, 0), (1, 2), (5, 0), (6, 0)])
+@pytest.mark.parametrize("M,N,K,planar", [(192, 24500, 2816, False), (192, 24500, 3072, True), (257, 16300, 1792, False),
+                                          (320, 16300, 2048, True), (321, 16300, 1024, True), (960, 6100, 768, False),
+                                          (960, 6100, 1024, True), (64, 49100, 1024, True)])
+def test_byte_types_route_by_last_row_tile(dev, wtype, atype, M, N, K, planar):
+    """384 workgroups of 128 x 128 with at most 64 rows in the last of several row tiles, of which the
+    LDS-DMA GEMM would compute 128, run there only with longer rows (two, three, eight row tiles; 65
+    rows and a single row tile: as full ones)."""
+    import torch
+    from ksq import ops
+    w = torch.zeros(N * (K // 32) * {1: 34, 5: 22, 6: 24}[wtype], dtype=torch.uint8, device=dev)
+    ops.gemm(wtype, atype, w, torch.ones(M, K, device=dev), M, N, K)
+    assert ops.last_engines() == {"quantize", "mmq_planar" if planar else "mmq6"}
+    torch.cuda.synchronize()
+
+
 @pytest.mark.parametrize("wtype,atype,M,N,K", [(wt, at, M, N, K) for wt, at in ((1, 0), (1, 2), (5, 0), (6, 0))
                                                for M, N, K in ((1500, 3100, 256), (1000, 5000, 4096), (65, 48000, 1536),
-                                                               (130, 24500, 1024), (1500, 4100, 512))])
+                                                               (130, 24500, 1024), (193, 24500, 1024),
+                                                               (130, 24500, 3072), (1500, 4100, 512))])
 def test_byte_types_result_independent_of_workspace(dev, wtype, atype, M, N, K):
     """The same call with the block form's workspace, with one that holds the planar form, from the
     library's pool and from the static scratch: the same bits (ordinary values, whose sums
