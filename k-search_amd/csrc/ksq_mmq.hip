@@ -1595,11 +1595,13 @@ hipError_t launch_mmq(int wtype, int afmt, const uint8_t* W, const uint8_t* A, f
 //    ahead by 4-15%) and from 1024 past that; one row tile is never behind.  Over 3400 shapes of
 //    388 .. 1008 workgroups, K = 512 .. 7168, Q8_0 and Q5_0.
 //  * 300 .. 383 workgroups, Q8_0: the pick is the 64 x 64 tile, 768 workgroups at a time and half
-//    the rows of padding, so it loses only where its grid needs well over one such round.  Past 1.5
-//    rounds from K = 4096 on (M = 1000, N = 5000 106 vs 88, M = 330, N = 14336 89.7 vs 87.7; K = 2048
-//    49.4 vs 52.0, M = 1500, N = 3100, K = 1024 30.5 vs 33.6; at 1.4 rounds M = 300, N = 14336, K = 4096
-//    86.0 vs 87.6), past 1.8 from K = 1536 (M = 1280, N = 4800 46.6 vs 44.1; K = 1024 35.4 vs 34.7, M =
-//    1299, N = 4352, K = 1024 32.8 vs 34.9).  One round: M = 40, N = 40000, K = 2048 30.3 vs 49.1.
+//    the rows of padding, so it loses only where its grid goes well into a second such round and the
+//    rows are long; most where they are a multiple of 2048 elements, on which it is itself slow (cause
+//    not traced).  Medians (least) of pick / this kernel over 3600 shapes: K = 4096, 6144, 8192 past
+//    1.5 rounds 1.06 (0.98) (M = 1000, N = 5000, K = 4096 106 vs 88 us), at 1.4 level or behind; K =
+//    2048 past 1.8 1.07 (0.97); other K from 4096 on past 1.65 1.03 (0.95), at 1.6 0.98 (0.93); from
+//    2304 to 3584 past 1.95 1.03 (0.94), at 1.8 1.01 (0.93); K = 1792 and below 1.00 (0.89: M = 328, N =
+//    15360, K = 1536 38.5 vs 43.4).
 //  * Q5_0 and Q5_1 not below 384: that pick adds the s_a term once per 8 blocks, this kernel (as the
 //    128 x 128 pick) per 4, and a result must not depend on whether the caller's workspace holds
 //    the planar form.
@@ -1620,8 +1622,9 @@ bool mmq_planar_preferred(int wtype, int M, int N, int K) {
         return K >= (wtype != kWQ80 ? 512 : wgs > 512 ? 768 : 1024);
     }
     if (wtype != kWQ80 || wgs < 300) return false;
-    const int round = kCUCount * TileS::OCC, wgs64 = grid_wgs<TileS>(M, N);
-    return (K >= 4096 && 2 * wgs64 > 3 * round) || (K >= 1536 && 5 * wgs64 > 9 * round);
+    const int percent = 100 * grid_wgs<TileS>(M, N) / (kCUCount * TileS::OCC);   // of a round
+    if (K % 2048 == 0) return percent >= (K >= 4096 ? 150 : 180);
+    return K >= 2048 && percent >= (K >= 4096 ? 165 : 195);
 }
 
 int mmq_planar_splits(int wtype, int M, int N, int K) { return split_for<TileL>(wtype, M, N, K); }

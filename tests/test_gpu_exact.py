@@ -258,9 +258,9 @@ def _engine_cases():
         cases.append((f"mmqp_auto_384_last2_w{wt}", wt, 130, 24500, 1024, 0, 0, 0, {"quantize", "mmq6"}, 0))
     # Q8_0 (also by block_q8s rules) below 384 where the 64 x 64 grid needs 1.8 rounds of the chip;
     # the K-step-8 sums of Q5 keep those on the 64 x 64 tile
-    cases.append(("mmqp_auto_375_w1", 1, 65, 48000, 1536, 0, 0, 0, {"quantize", "mmq_planar"}, 0))
-    cases.append(("mmqp_auto_375_q8s", 1, 65, 48000, 1536, 2, 0, 0, {"quantize", "mmq_planar"}, 0))
-    cases.append(("mmqp_auto_375_w5", 5, 65, 48000, 1536, 0, 0, 0, {"quantize", "mmq3"}, 0))
+    cases.append(("mmqp_auto_375_w1", 1, 65, 48000, 2048, 0, 0, 0, {"quantize", "mmq_planar"}, 0))
+    cases.append(("mmqp_auto_375_q8s", 1, 65, 48000, 2048, 2, 0, 0, {"quantize", "mmq_planar"}, 0))
+    cases.append(("mmqp_auto_375_w5", 5, 65, 48000, 2048, 0, 0, 0, {"quantize", "mmq3"}, 0))
     cases.append(("splitk_w0", 0, 32, 1024, 8192, 1, 2, 0, {"mmq5", "splitk"}, 0))
     cases.append(("splitk_w1", 1, 32, 1024, 8192, 1, 2, 0, {"mmq3", "splitk"}, 0))
     # the native W8A8C8 operator's block_q8s activations: fp32 (its quantiser) and pre-quantised
@@ -557,8 +557,24 @@ def test_byte_types_route_by_last_row_tile(dev, wtype, atype, M, N, K, planar):
     torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("atype", [0, 2])
+@pytest.mark.parametrize("M,N,K,planar", [(328, 15360, 1536, False), (328, 15360, 1792, False), (328, 15360, 2048, True),
+                                          (328, 15360, 2560, False), (512, 12032, 2304, True), (250, 19200, 3584, False),
+                                          (300, 14336, 4096, False), (330, 14336, 4096, True), (1000, 5000, 4096, True),
+                                          (1000, 5000, 4608, False), (640, 8960, 4608, True)])
+def test_q8_0_route_below_384_workgroups(dev, atype, M, N, K, planar):
+    """300 to 383 workgroups of 128 x 128: the LDS-DMA GEMM where the 64 x 64 grid goes well into a
+    second round of the chip and the rows are long, or a multiple of 2048 elements."""
+    import torch
+    from ksq import ops
+    w = torch.zeros(N * (K // 32) * 34, dtype=torch.uint8, device=dev)
+    ops.gemm(1, atype, w, torch.ones(M, K, device=dev), M, N, K)
+    assert ops.last_engines() == {"quantize", "mmq_planar" if planar else "mmq3"}
+    torch.cuda.synchronize()
+
+
 @pytest.mark.parametrize("wtype,atype,M,N,K", [(wt, at, M, N, K) for wt, at in ((1, 0), (1, 2), (5, 0), (6, 0))
-                                               for M, N, K in ((1500, 3100, 256), (1000, 5000, 4096), (65, 48000, 1536),
+                                               for M, N, K in ((1500, 3100, 256), (1000, 5000, 4096), (65, 48000, 2048),
                                                                (130, 24500, 1024), (193, 24500, 1024),
                                                                (130, 24500, 3072), (1500, 4100, 512))])
 def test_byte_types_result_independent_of_workspace(dev, wtype, atype, M, N, K):
