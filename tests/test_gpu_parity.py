@@ -518,7 +518,7 @@ def test_moe_config4_sampled(dev, oracle):
 @pytest.mark.parametrize("wtype", ALL_WTYPES)
 def test_mfma_tile_configs(dev, oracle, cfg, wtype):
     """Every MFMA tile configuration (K step 4 is not used for K-quants: they take the automatic tile;
-    configuration 8 is the LDS-DMA GEMM for Q4_0 / Q4_1, the 128 x 128 tile for the rest)."""
+    configuration 8 is the LDS-DMA GEMM for the 32-element types, the 128 x 128 tile for K-quants)."""
     from ksq import _lib, synth
     g = np.random.default_rng(1500 + 10 * cfg + wtype)
     M, N, K = 150, 136, 512
